@@ -55,12 +55,12 @@ struct PyrView {
 // textureLod with LINEAR_MIPMAP_LINEAR on an isotropic pyramid (border 0).
 __device__ __forceinline__ float4 sample_iso(const PyrView &v, const float p[3], float lam) {
     const int q = v.nlevels - 1;
-    if (!(lam < (float)q)) return level_linear(v.pyr, v.scales, v.lv[q], p);
+    if (!(lam < (float)q)) return level_linear(v.pyr, v.lv[q], p);
     if (lam < 0.0f) lam = 0.0f;
     int d1 = (int)floorf(lam);
     d1 = d1 > q - 1 ? q - 1 : d1;
     const float fr = lam - (float)d1;
-    const float4 a = level_linear(v.pyr, v.scales, v.lv[d1], p), b = level_linear(v.pyr, v.scales, v.lv[d1 + 1], p);
+    const float4 a = level_linear(v.pyr, v.lv[d1], p), b = level_linear(v.pyr, v.lv[d1 + 1], p);
     return make_float4((1.0f - fr) * a.x + fr * b.x, (1.0f - fr) * a.y + fr * b.y, (1.0f - fr) * a.z + fr * b.z,
                        (1.0f - fr) * a.w + fr * b.w);
 }
@@ -1113,7 +1113,7 @@ __global__ __launch_bounds__(256) void k_learned_fallback(TraceLaunch t, PyrArgs
     for (uint32_t i = blockIdx.x * 4 + (threadIdx.x >> 6); i < n; i += gridDim.x * 4) {
         const int tile = (int)list[1 + i];
         const int px = (tile % tiles_x) * 8 + (lane & 7), py = (tile / tiles_x) * 8 + (lane >> 3);
-        if (px < t.width && py < t.height) trace_pixel<MODE, false>(t, pa, pyr_rsrc(pa), px, py, false);
+        if (px < t.width && py < t.height) trace_pixel<MODE, false, false>(t, pa, pyr_rsrc(pa), px, py, false);
     }
 }
 

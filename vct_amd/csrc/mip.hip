@@ -262,6 +262,12 @@ __global__ __launch_bounds__(256) void k_mip_chain(MipArgs a) {
 
 // FP8 E4M3 encode of one level: one 64-thread wavefront per (brick, face);
 // the scale is the largest magnitude in the brick over 448 (1 if all zero).
+// The chain is done with the level's stage by now, so the decoded texels
+// (code * scale, what load_texel returns) take its place as fp32 elements,
+// with zeros in the border element of texel -1 (the second half of which held
+// texel 0 of an fp16 pair): the trace reads a texel with one 16-byte load and
+// no decoding, which it would otherwise repeat for every corner of every
+// sample.
 __global__ __launch_bounds__(64) void k_fp8_encode(char *pyr, float *scales, LevelInfo L) {
     const int bf = blockIdx.x;  // brick * nfaces + face
     const int b = bf / L.nfaces, f = bf % L.nfaces;
@@ -279,6 +285,9 @@ __global__ __launch_bounds__(64) void k_fp8_encode(char *pyr, float *scales, Lev
     if (v == 0) scales[L.scale + (e >> 6)] = sc;
     const uint32_t code = f2fp8(c.x / sc) | (f2fp8(c.y / sc) << 8) | (f2fp8(c.z / sc) << 16) | (f2fp8(c.w / sc) << 24);
     *(uint32_t *)(pyr + L.base + (size_t)e * 4) = code;
+    *(float4 *)(pyr + L.stage + (size_t)e * 16) = decode_fp8x4(code, sc);
+    if (x == 0)  // the element index of x = -1 wraps below 0: the byte offset is formed in 32 bits
+        *(float4 *)(pyr + (uint32_t)(L.stage + elem_index(L, -1, y, z, f) * 16u)) = make_float4(0.f, 0.f, 0.f, 0.f);
 }
 
 // ---------------------------------------------------------------- albedo chain

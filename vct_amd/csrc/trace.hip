@@ -13,7 +13,7 @@
 
 namespace vctk {
 
-template <int MODE, bool ANISO>
+template <int MODE, bool ANISO, bool WARP>
 __global__ __launch_bounds__(256) void k_trace(TraceLaunch t, PyrArgs pa, int tiles_x, int tiles, int per_xcd) {
     // XCD-aware tile order: workgroup b runs on XCD b % 8; give XCD k the
     // contiguous tile band [k * per_xcd, (k + 1) * per_xcd).
@@ -24,7 +24,7 @@ __global__ __launch_bounds__(256) void k_trace(TraceLaunch t, PyrArgs pa, int ti
     const int px = (tile % tiles_x) * 16 + (wave & 1) * 8 + (lane & 7);
     const int py = (tile / tiles_x) * 16 + (wave >> 1) * 8 + (lane >> 3);
     if (px >= t.width || py >= t.height) return;
-    trace_pixel<MODE, ANISO>(t, pa, pyr_rsrc(pa), px, py, t.enable_reflections != 0);
+    trace_pixel<MODE, ANISO, WARP>(t, pa, pyr_rsrc(pa), px, py, t.enable_reflections != 0);
 }
 
 hipError_t launch_trace(const PyrDesc &pyr, const TraceLaunch &t, hipStream_t s) {
@@ -33,17 +33,22 @@ hipError_t launch_trace(const PyrDesc &pyr, const TraceLaunch &t, hipStream_t s)
     const int per_xcd = (tiles + 7) / 8;
     dim3 grid((unsigned)(per_xcd * 8));
     const int mode = pyr.storage == VCT_STORE_FP32 ? 1 : (pyr.storage == VCT_STORE_FP8 ? 2 : 0);
-#define VCT_TRACE_LAUNCH(M, A)                                                                                      \
-    hipLaunchKernelGGL((k_trace<M, A>), grid, dim3(256), 0, s, t, pyr_args(pyr, t.nested), tiles_x, tiles, per_xcd)
-    if (pyr.aniso) {
-        if (mode == 0) VCT_TRACE_LAUNCH(0, true);
-        else if (mode == 1) VCT_TRACE_LAUNCH(1, true);
-        else VCT_TRACE_LAUNCH(2, true);
+#define VCT_TRACE_LAUNCH(M, A, W)                                                                                   \
+    hipLaunchKernelGGL((k_trace<M, A, W>), grid, dim3(256), 0, s, t, pyr_args(pyr, t.nested), tiles_x, tiles, per_xcd)
+#define VCT_TRACE_MODES(A, W)                 \
+    if (mode == 0) VCT_TRACE_LAUNCH(0, A, W);      \
+    else if (mode == 1) VCT_TRACE_LAUNCH(1, A, W); \
+    else VCT_TRACE_LAUNCH(2, A, W)
+    if (pyr.aniso && t.warp) {
+        VCT_TRACE_MODES(true, true);
+    } else if (pyr.aniso) {
+        VCT_TRACE_MODES(true, false);
+    } else if (t.warp) {
+        VCT_TRACE_MODES(false, true);
     } else {
-        if (mode == 0) VCT_TRACE_LAUNCH(0, false);
-        else if (mode == 1) VCT_TRACE_LAUNCH(1, false);
-        else VCT_TRACE_LAUNCH(2, false);
+        VCT_TRACE_MODES(false, false);
     }
+#undef VCT_TRACE_MODES
 #undef VCT_TRACE_LAUNCH
     return hipGetLastError();
 }

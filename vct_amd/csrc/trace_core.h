@@ -19,20 +19,19 @@ namespace vctk {
 // element index is a sum of per-axis terms (vct_internal.h):
 //   X(x) = (x>>2)*sx + (x&3),  Y(y) = (y>>2)*sy + (y&3)*4,
 //   Z(z) = (z>>2)*sz + (z&3)*16, plus 64 per face.
-// fp16 levels read corners outside the level (the border) from the zero
-// border bricks around every level; the one-texel-per-element formats clamp
-// them to a valid texel with weight 0.  Either way all fetches are
-// unconditional.  fp16 levels store texel pairs
-// (x, x+1) per element: a trilinear sample is four 16-byte loads, one per
-// (y, z) corner pair, instead of eight 8-byte loads -- the vector memory
+// Corners outside the level (the border) are read from the zero border bricks
+// around every level, so all fetches are unconditional.  fp16 levels store
+// texel pairs (x, x+1) per element: a trilinear sample is four 16-byte loads,
+// one per (y, z) corner pair, instead of eight 8-byte loads -- the vector memory
 // pipeline processes a wavefront's load in the same number of cycles for 8 or
-// 16 bytes per lane, so this halves the trace's dominant cost.
+// 16 bytes per lane, so this halves the trace's dominant cost.  fp32 levels, and
+// fp8 levels in their decoded copy (LevelInfo::stage, written by the encoder),
+// hold one 16-byte texel per element: eight loads.
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 struct PyrArgs {
     const char *pyr;
     uint32_t bytes;
-    const float *scales;
     const LevelInfo *lv;
     int dim, nlevels;
     int nested;  // TraceLaunch::nested
@@ -41,9 +40,6 @@ struct PyrArgs {
 __device__ __forceinline__ uint4 bload16(__amdgpu_buffer_rsrc_t r, uint32_t off) {
     const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(r, (int)off, 0, 0);
     return make_uint4(v.x, v.y, v.z, v.w);
-}
-__device__ __forceinline__ uint32_t bload4(__amdgpu_buffer_rsrc_t r, uint32_t off) {
-    return __builtin_amdgcn_raw_buffer_load_b32(r, (int)off, 0, 0);
 }
 // Scalar load of 16 bytes at a wave-uniform offset: through the constant
 // address space the load becomes s_load_dwordx4 into SGPRs (scalar data cache,
@@ -56,35 +52,61 @@ __device__ __forceinline__ uint4 sload16(const char *pyr, uint32_t off) {
     return make_uint4(v.x, v.y, v.z, v.w);
 }
 
-__device__ __forceinline__ void axis_terms(float p, int s, uint32_t mul, uint32_t sub, uint32_t t[2], float w[2]) {
-    const float u = p * (float)s - 0.5f;
-    const float fl = __builtin_floorf(u);
-    const int i0 = (int)fl;
-    const float f = u - fl;
-    const int i1 = i0 + 1;
-    w[0] = (i0 >= 0) ? 1.0f - f : 0.0f;  // i0 <= s - 1 always (p <= 1)
-    w[1] = (i1 < s) ? f : 0.0f;          // i1 >= 0 always (p >= 0)
-    const int c0 = i0 < 0 ? 0 : i0, c1 = i1 > s - 1 ? s - 1 : i1;
-    // brick index < 2^7 and stride < 2^24 (dim <= 512): full-rate 24-bit multiplies
-    t[0] = __umul24((uint32_t)(c0 >> 2), mul) + (uint32_t)(c0 & 3) * sub;
-    t[1] = __umul24((uint32_t)(c1 >> 2), mul) + (uint32_t)(c1 & 3) * sub;
+// warp_sample (vct_device.h) for the march: at 1080p and above a wavefront's
+// positions nearly always lie in one cell of the 32^3 texture, whose eight
+// texels then come through scalar loads (the texture is not written while a
+// trace runs); the per-lane form fetches eight float4 per step and lane.  The
+// same products and sums in the same order, so both forms agree bit for bit.
+__device__ __forceinline__ void warp_sample_march(const float4 *__restrict__ wm, float p[3]) {
+    int i0[3], i1[3];
+    float f[3];
+    bool same = true;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        const float u = p[k] * (float)kWarpDim - 0.5f;
+        const float fl = __builtin_floorf(u);
+        f[k] = u - fl;
+        const int a = (int)fl;
+        same = same && __builtin_amdgcn_readfirstlane(a) == a;
+        i0[k] = a < 0 ? 0 : (a > kWarpDim - 1 ? kWarpDim - 1 : a);
+        i1[k] = a + 1 < 0 ? 0 : (a + 1 > kWarpDim - 1 ? kWarpDim - 1 : a + 1);
+    }
+    if (__ballot(same) != __ballot(true)) {
+        warp_sample(wm, p, p);
+        return;
+    }
+    float acc[3] = {0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int c = 0; c < 8; ++c) {
+        const int dx = c & 1, dy = (c >> 1) & 1, dz = c >> 2;
+        const float w = ((dx ? f[0] : 1.0f - f[0]) * (dy ? f[1] : 1.0f - f[1])) * (dz ? f[2] : 1.0f - f[2]);
+        const uint32_t e = (uint32_t)(((dz ? i1[2] : i0[2]) * kWarpDim + (dy ? i1[1] : i0[1])) * kWarpDim +
+                                      (dx ? i1[0] : i0[0]));
+        const uint4 t = sload16((const char *)wm, __builtin_amdgcn_readfirstlane(e) * 16u);
+        acc[0] = acc[0] + w * __uint_as_float(t.x);
+        acc[1] = acc[1] + w * __uint_as_float(t.y);
+        acc[2] = acc[2] + w * __uint_as_float(t.z);
+    }
+#pragma unroll
+    for (int k = 0; k < 3; ++k) p[k] = acc[k];
 }
-
 
 // All 2x2x2 texels of a uniform fetch are +0 (empty space): their weighted sum
 // adds exactly 0, so the weighting is skipped.  The test runs on the scalar
 // unit, beside the vector work of the other wavefronts.
-__device__ __forceinline__ bool zero16(const uint4 v[4]) {
+template <int N>
+__device__ __forceinline__ bool zero16(const uint4 (&v)[N]) {
     uint32_t o = 0u;
 #pragma unroll
-    for (int c = 0; c < 4; ++c) o |= (v[c].x | v[c].y) | (v[c].z | v[c].w);
+    for (int c = 0; c < N; ++c) o |= (v[c].x | v[c].y) | (v[c].z | v[c].w);
     return o == 0u;
 }
 
-// The fp16-pair sampler's axis terms: the border bricks hold texels -1 and s
-// as zeros, so neither index is clamped nor weight masked.  Indices are
-// shifted by one brick (+4, never negative for the 24-bit multiplies) and
-// offsets are taken from the level's storage start.
+// The sampler's axis terms: the border bricks hold texels -1 and s as zeros,
+// so neither index is clamped nor weight masked.  Indices are shifted by one
+// brick (+4, never negative for the 24-bit multiplies; brick index < 2^7 + 2,
+// stride < 2^24 for dim <= 512) and offsets are taken from the level's storage
+// start.
 __device__ __forceinline__ void axis_terms_pad(float p, int s, uint32_t mul, uint32_t sub, uint32_t t[2], float w[2]) {
     const float u = p * (float)s - 0.5f;
     const float fl = __builtin_floorf(u);
@@ -119,62 +141,107 @@ __device__ __forceinline__ void acc_f4(float4 &acc, uint4 v, float w) {
     acc.w = fmaf(__uint_as_float(v.w), w, acc.w);
 }
 
+// acc += lw * (trilinear sample of level L at p), for levels of one 16-byte
+// fp32 texel per element (fp32 storage; the decoded copy of an fp8 level).  The
+// arguments and the wave-uniform scalar path are those of level_sample below.
+// The offsets of the eight corners are sums of the axis terms, formed as they
+// are used.  Bound by VALU issue in the scalar path (40 instructions per face)
+// and by the texture-address unit in the per-lane one (eight loads per face).
+// Measured: the FP8 trace of the 3840x2160 warped scene 28.9 -> 9 ms and of a
+// 961x541 frame 1.72 -> 0.55 ms against four-byte loads decoded per corner
+// (their decoder made the sampler a called function with scratch memory); the
+// isotropic FP32 gather at 1001x567 242 -> 223 us.  Texels are weighted and
+// summed in one fixed order (w[k] * d2 into acc): a march compares its opacity
+// with 0.95, and sums that differ in the last bit end some cones a step apart.
+template <bool ZQ>
+__device__ __forceinline__ bool level_sample_f32(float4 &acc, const char *pyr, __amdgpu_buffer_rsrc_t rs,
+                                                 const LevelInfo &L, const float p[3], float lw, const uint32_t fe[3],
+                                                 const float d2[3], uint32_t fmask, bool fsame) {
+    const int s = L.size;
+    const bool aniso = L.nfaces == 6;
+    uint32_t tx[2], ty[2], tz[2];
+    float wx[2], wy[2], wz[2];
+    axis_terms_pad(p[0], s, L.sx, 1u, tx, wx);
+    axis_terms_pad(p[1], s, L.sy, 4u, ty, wy);
+    axis_terms_pad(p[2], s, L.sz, 16u, tz, wz);
+    const uint32_t org = L.stage - L.pad * 16u;  // the level's storage start
+    wz[0] *= lw;
+    wz[1] *= lw;
+    float w[8];
+    uint32_t oyz[4];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+        w[2 * c] = (wx[0] * wy[c & 1]) * wz[c >> 1];
+        w[2 * c + 1] = (wx[1] * wy[c & 1]) * wz[c >> 1];
+        oyz[c] = org + (ty[c & 1] + tz[c >> 1]) * 16u;
+    }
+    const uint32_t o0 = oyz[0] + tx[0] * 16u, o7 = oyz[3] + tx[1] * 16u;
+    const bool same = (!aniso || fsame) && __builtin_amdgcn_readfirstlane(o0) == o0 &&
+                      __builtin_amdgcn_readfirstlane(o7) == o7;
+    const int nf = aniso ? 3 : 1;
+    if (__ballot(same) == __ballot(true)) {
+        const uint32_t sx0 = __builtin_amdgcn_readfirstlane(tx[0]) * 16u, sx1 = __builtin_amdgcn_readfirstlane(tx[1]) * 16u;
+        uint32_t so[4];
+#pragma unroll
+        for (int c = 0; c < 4; ++c) so[c] = __builtin_amdgcn_readfirstlane(oyz[c]);
+        bool z = true;
+        for (int a = 0; a < nf; ++a) {
+            if (aniso && !((fmask >> a) & 1u)) continue;
+            const uint32_t fo = aniso ? __builtin_amdgcn_readfirstlane(fe[a]) * 16u : 0u;
+            uint4 v[8];
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                v[2 * c] = sload16(pyr, so[c] + sx0 + fo);
+                v[2 * c + 1] = sload16(pyr, so[c] + sx1 + fo);
+            }
+            if (zero16(v)) continue;
+            z = false;
+            const float fw = aniso ? d2[a] : 1.0f;
+#pragma unroll
+            for (int k = 0; k < 8; ++k) acc_f4(acc, v[k], w[k] * fw);
+        }
+        return z;
+    }
+    bool z = ZQ;
+    for (int a = 0; a < nf; ++a) {
+        if (aniso && !((fmask >> a) & 1u)) continue;
+        const uint32_t fo = aniso ? fe[a] * 16u : 0u;
+        uint4 v[8];
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            v[2 * c] = bload16(rs, oyz[c] + tx[0] * 16u + fo);
+            v[2 * c + 1] = bload16(rs, oyz[c] + tx[1] * 16u + fo);
+        }
+        if (ZQ && __ballot(!zero16(v)) == 0) continue;
+        z = false;
+        const float fw = aniso ? d2[a] : 1.0f;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) acc_f4(acc, v[k], w[k] * fw);
+    }
+    return z;
+}
+
 // acc += lw * (trilinear sample of level L at p): isotropic, or the
 // dir^2-weighted mix of the three faces that face the cone (fe: their element
 // offsets, 64 * face).  L is wave-uniform.  fmask (wave-uniform) has bit a
 // set unless d2[a] is 0 in every lane: a face no lane weights adds exactly 0
 // and is not fetched.  Returns (wave-uniform) whether every texel fetched, in
-// every lane, was +0 -- reported by the fp16 paths only (ZQ: also test the
-// per-lane fetches, which costs vector instructions).
+// every lane, was +0 (ZQ: also test the per-lane fetches, which costs vector
+// instructions).  An fp8 level reports false: its codes underflow, so a zero
+// there does not say that the finer level is zero.
 template <int MODE, bool ZQ>
 __device__ __forceinline__ bool level_sample(float4 &acc, const char *pyr, __amdgpu_buffer_rsrc_t rs,
-                                             const float *__restrict__ scales, const LevelInfo &L, const float p[3],
-                                             float lw, const uint32_t fe[3], const float d2[3], uint32_t fmask,
-                                             bool fsame) {
+                                             const LevelInfo &L, const float p[3], float lw, const uint32_t fe[3],
+                                             const float d2[3], uint32_t fmask, bool fsame) {
+    if (MODE == 1) return level_sample_f32<ZQ>(acc, pyr, rs, L, p, lw, fe, d2, fmask, fsame);
+    if (MODE == 2 && L.fmt == 2) {
+        level_sample_f32<false>(acc, pyr, rs, L, p, lw, fe, d2, fmask, fsame);
+        return false;
+    }
     const int s = L.size;
     const bool aniso = L.nfaces == 6;
     uint32_t ty[2], tz[2];
     float wy[2], wz[2];
-    if (MODE == 1 || (MODE == 2 && L.fmt == 2)) {  // one texel per element: 8 corners
-        axis_terms(p[1], s, L.sy, 4u, ty, wy);
-        axis_terms(p[2], s, L.sz, 16u, tz, wz);
-        wz[0] *= lw;
-        wz[1] *= lw;
-        uint32_t tx[2];
-        float wx[2];
-        axis_terms(p[0], s, L.sx, 1u, tx, wx);
-        uint32_t e[8];
-        float w[8];
-#pragma unroll
-        for (int k = 0; k < 8; ++k) {
-            const int dx = k & 1, dy = (k >> 1) & 1, dz = k >> 2;
-            e[k] = tx[dx] + ty[dy] + tz[dz];
-            w[k] = (wx[dx] * wy[dy]) * wz[dz];
-        }
-        const int nf = aniso ? 3 : 1;
-        for (int a = 0; a < nf; ++a) {
-            if (aniso && !((fmask >> a) & 1u)) continue;
-            const uint32_t fo = aniso ? fe[a] : 0u;
-            const float fw = aniso ? d2[a] : 1.0f;
-            if (MODE == 1) {
-#pragma unroll
-                for (int k = 0; k < 8; ++k) acc_f4(acc, bload16(rs, L.base + (e[k] + fo) * 16u), w[k] * fw);
-            } else {
-#pragma unroll
-                for (int k = 0; k < 8; ++k) {
-                    const uint32_t ee = e[k] + fo;
-                    const uint32_t c = bload4(rs, L.base + ee * 4u);
-                    const float4 t = decode_fp8x4(c, scales[L.scale + (ee >> 6)]);
-                    const float ww = w[k] * fw;
-                    acc.x = fmaf(t.x, ww, acc.x);
-                    acc.y = fmaf(t.y, ww, acc.y);
-                    acc.z = fmaf(t.z, ww, acc.z);
-                    acc.w = fmaf(t.w, ww, acc.w);
-                }
-            }
-        }
-        return false;
-    }
     // fp16 pairs: element x holds texels x and x+1, so one load per (y, z)
     // corner pair; element -1 (border brick) holds (0, texel 0)
     axis_terms_pad(p[1], s, L.sy, 4u, ty, wy);
@@ -310,7 +377,7 @@ __device__ __forceinline__ float4 sample_class(const PyrArgs &pa, __amdgpu_buffe
         return unpack_h4(v.x, v.y);
     }
     if (D >= q) {
-        level_sample<MODE, false>(acc, pa.pyr, rs, pa.scales, pa.lv[q], p, 1.0f, fe, d2, fmask, fsame);
+        level_sample<MODE, false>(acc, pa.pyr, rs, pa.lv[q], p, 1.0f, fe, d2, fmask, fsame);
         return acc;
     }
     // The coarser level first.  Its 2x2x2 cell covers the finer level's cell
@@ -319,9 +386,9 @@ __device__ __forceinline__ float4 sample_class(const PyrArgs &pa, __amdgpu_buffe
     // is zero only where every texel it filters is.  So where the coarser
     // fetch was all zero in every lane, the finer sample adds exactly 0 and is
     // skipped: cones marching through empty space.
-    const bool z = level_sample<MODE, true>(acc, pa.pyr, rs, pa.scales, pa.lv[D + 1], p, fr, fe, d2, fmask, fsame);
+    const bool z = level_sample<MODE, true>(acc, pa.pyr, rs, pa.lv[D + 1], p, fr, fe, d2, fmask, fsame);
     if (!(z && pa.nested))
-        level_sample<MODE, false>(acc, pa.pyr, rs, pa.scales, pa.lv[D], p, 1.0f - fr, fe, d2, fmask, fsame);
+        level_sample<MODE, false>(acc, pa.pyr, rs, pa.lv[D], p, 1.0f - fr, fe, d2, fmask, fsame);
     return acc;
 }
 
@@ -332,9 +399,11 @@ __device__ __forceinline__ float4 sample_class(const PyrArgs &pa, __amdgpu_buffe
 // cones, whose schedule the host computed for the launch), read from the
 // kernel arguments.  Otherwise the lanes' level classes are visited one at a
 // time (each pass with a uniform class).
-// warp: warpTexture (phong.frag:150-152), each sample position goes through the
-// warp texture before the pyramid is sampled (the level stays the unwarped one).
-template <int MODE, bool ANISO, bool ULOD>
+// WARP: warpTexture (phong.frag:150-152), each sample position goes through the
+// warp texture before the pyramid is sampled (the level stays the unwarped
+// one); a template argument, since the registers it takes would cost the
+// unwarped tracer a wavefront per SIMD.
+template <int MODE, bool ANISO, bool ULOD, bool WARP>
 __device__ float4 trace_cone(const PyrArgs &pa, __amdgpu_buffer_rsrc_t rs, const float pos[3], const float nrm[3],
                              const float dir_in[3], int steps, float bias, float tan_half, float h0,
                              float lod_offset, const float4 *warp, const ConeSchedule *sched = nullptr) {
@@ -378,7 +447,7 @@ __device__ float4 trace_cone(const PyrArgs &pa, __amdgpu_buffer_rsrc_t rs, const
 #pragma unroll
             for (int k = 0; k < 3; ++k) sp[k] = start[k] + h * ds[k];
             if (sp[0] < 0.f || sp[0] > 1.f || sp[1] < 0.f || sp[1] > 1.f || sp[2] < 0.f || sp[2] > 1.f) break;
-            if (warp) warp_sample(warp, sp, sp);
+            if (WARP) warp_sample_march(warp, sp);
             const float4 smp = sample_class<MODE>(pa, rs, sched->cls[i], sched->fr[i], sp, fe, d2, fmask, fsame);
             const float aa = 1.0f - a;
             c0 += smp.x * aa;
@@ -396,7 +465,7 @@ __device__ float4 trace_cone(const PyrArgs &pa, __amdgpu_buffer_rsrc_t rs, const
 #pragma unroll
         for (int k = 0; k < 3; ++k) sp[k] = start[k] + (h * dir[k]) * scale;
         if (sp[0] < 0.f || sp[0] > 1.f || sp[1] < 0.f || sp[1] > 1.f || sp[2] < 0.f || sp[2] > 1.f) break;
-        if (warp) warp_sample(warp, sp, sp);
+        if (WARP) warp_sample_march(warp, sp);
         float fr;
         const int D = level_class(lod + lod_offset, q, &fr);
         float4 smp;
@@ -436,7 +505,7 @@ static __constant__ float kConeDirs[6][3] = {{0.0f, 1.0f, 0.0f},
 static __constant__ float kConeW[6] = {0.25f, 0.15f, 0.15f, 0.15f, 0.15f, 0.15f};
 
 // One pixel of the phong.frag gather: 6 diffuse cones (+ the specular cone).
-template <int MODE, bool ANISO>
+template <int MODE, bool ANISO, bool WARP>
 __device__ __forceinline__ void trace_pixel(const TraceLaunch &t, const PyrArgs &pa, __amdgpu_buffer_rsrc_t rs, int px,
                                             int py, bool reflections) {
     const size_t pi = (size_t)py * t.width + px;
@@ -462,7 +531,7 @@ __device__ __forceinline__ void trace_pixel(const TraceLaunch &t, const PyrArgs 
         float d[3];
 #pragma unroll
         for (int k = 0; k < 3; ++k) d[k] = (T[k] * cx + B[k] * cy) + nraw[k] * cz;
-        const float4 r = trace_cone<MODE, ANISO, true>(pa, rs, pos, N, d, t.d_steps, t.d_bias, t.d_tan_half, t.d_h0,
+        const float4 r = trace_cone<MODE, ANISO, true, WARP>(pa, rs, pos, N, d, t.d_steps, t.d_bias, t.d_tan_half, t.d_h0,
                                                        t.d_lod_offset, t.warp, &t.d_sched);
         const float w = kConeW[i];
         i0 += w * r.x;
@@ -488,10 +557,10 @@ __device__ __forceinline__ void trace_pixel(const TraceLaunch &t, const PyrArgs 
         const float th0 = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(th)));
         float4 r;
         if (__ballot(__float_as_int(th) != __float_as_int(th0)) == 0)
-            r = trace_cone<MODE, ANISO, true>(pa, rs, pos, N, R, t.s_steps, t.s_bias, th, t.s_h0, t.s_lod_offset,
+            r = trace_cone<MODE, ANISO, true, WARP>(pa, rs, pos, N, R, t.s_steps, t.s_bias, th, t.s_h0, t.s_lod_offset,
                                               t.warp);
         else
-            r = trace_cone<MODE, ANISO, false>(pa, rs, pos, N, R, t.s_steps, t.s_bias, th, t.s_h0, t.s_lod_offset,
+            r = trace_cone<MODE, ANISO, false, WARP>(pa, rs, pos, N, R, t.s_steps, t.s_bias, th, t.s_h0, t.s_lod_offset,
                                                t.warp);
         t.out_spec[pi] = r;
     }
@@ -501,7 +570,6 @@ inline PyrArgs pyr_args(const PyrDesc &pyr, int nested) {
     PyrArgs a;
     a.pyr = pyr.pyr;
     a.bytes = pyr.bytes;
-    a.scales = pyr.scales;
     a.lv = pyr.d_lv;
     a.dim = pyr.dim;
     a.nlevels = pyr.nlevels;

@@ -226,7 +226,7 @@ __device__ __forceinline__ float4 load_texel(const char *pyr, const float *scale
 
 // GL LINEAR inside face 0 of one level (border 0), FP32 weights and sums.
 // p in [0,1]^3 texture coordinates; s = the level's edge.
-__device__ __forceinline__ float4 level_linear(const char *pyr, const float *scales, const LevelInfo &L, const float p[3]) {
+__device__ __forceinline__ float4 level_linear(const char *pyr, const LevelInfo &L, const float p[3]) {
     const int s = L.size;
     int i0[3];
     float f[3];
@@ -263,7 +263,8 @@ __device__ __forceinline__ float4 level_linear(const char *pyr, const float *sca
         const int x = i0[0] + dx, y = i0[1] + dy, z = i0[2] + dz;
         if ((unsigned)x >= (unsigned)s || (unsigned)y >= (unsigned)s || (unsigned)z >= (unsigned)s) continue;
         const float w = ((dx ? f[0] : 1.0f - f[0]) * (dy ? f[1] : 1.0f - f[1])) * (dz ? f[2] : 1.0f - f[2]);
-        const float4 t = load_texel(pyr, scales, L, x, y, z, 0);
+        // fp32 elements, or the decoded copy of an fp8 level
+        const float4 t = *(const float4 *)(pyr + L.stage + (size_t)elem_index(L, x, y, z, 0) * 16);
         acc.x += w * t.x;
         acc.y += w * t.y;
         acc.z += w * t.z;

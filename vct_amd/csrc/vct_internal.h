@@ -43,7 +43,7 @@ struct DevLight {
 // volumes (1, or 6 for anisotropic levels >= 1: +x,-x,+y,-y,+z,-z).  A brick
 // holds 4x4x4 elements x-fastest and the faces of one brick are adjacent.
 // Every level carries a border one brick thick on each side (nb + 2 bricks
-// per axis) that holds zeros, so that the fp16-pair sampler can fetch texel
+// per axis) that holds zeros, so that the samplers can fetch texel
 // -1 and texel size of any axis without clamping or masking.  With `base` at
 // the first interior brick, the element of texel (x, y, z) in face f is
 //   (x>>2)*sx + (x&3) + (y>>2)*sy + (y&3)*4 + (z>>2)*sz + (z&3)*16 + 64*f
@@ -60,7 +60,9 @@ struct DevLight {
 //   2  fp8 E4M3 x4, 4 B, one texel, times the fp32 scale of its (brick, face):
 //      scales[scale + element / 64].
 // `stage` is where the mip chain reads and writes the level: `base` for fmt 0
-// and 1, an fp16-pair copy for fmt 2 (filtered in fp16, encoded after).
+// and 1, a copy for fmt 2: fp16 pairs while the chain runs, then, when the
+// level is encoded, the decoded texels as fp32x4 (fmt 1 elements), which the
+// samplers read.
 struct LevelInfo {
     uint32_t base, stage;  // byte offsets into the pyramid allocation (first interior brick)
     uint32_t scale;        // float offset into the scale array (fmt 2)
