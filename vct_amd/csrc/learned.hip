@@ -414,22 +414,6 @@ __global__ __launch_bounds__(256) void k_features(const vct_gbuffer_texel *__res
     make_features<FMT>(g[0], g[3], pv, ext, (uint32_t *)(X + (size_t)i * kMlpIn));
 }
 
-// ---------------------------------------------------------------- MFMA tiles
-// acc (16x16 tile at rows m0, cols n0) += A[m][k] * B[n][k] over k in [0, K),
-// A row-major with leading dimension lda, B "n-major" (each column's k-vector
-// contiguous) with leading dimension ldb; both BF16; K a multiple of 32.
-__device__ __forceinline__ f32x4 mfma_tile(const uint16_t *A, int lda, const uint16_t *B, int ldb, int m0, int n0,
-                                           int K, f32x4 acc) {
-    const int lane = threadIdx.x & 63;
-    const int r = lane & 15, kq = (lane >> 4) * 8;
-    for (int k0 = 0; k0 < K; k0 += 32) {
-        const bf16x8 a = *(const bf16x8 *)(A + (size_t)(m0 + r) * lda + k0 + kq);
-        const bf16x8 b = *(const bf16x8 *)(B + (size_t)(n0 + r) * ldb + k0 + kq);
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc, 0, 0, 0);
-    }
-    return acc;
-}
-
 // ---------------------------------------------------------------- training
 struct MlpDev {
     const float *master;  // [kMlpParams] FP32 (W1, b1, W2, b2, W3, b3, W4, b4; W row-major out x in)
@@ -459,173 +443,265 @@ __device__ __forceinline__ uint32_t mix_hash(uint32_t x) {
     return x;
 }
 
-// Shared memory of one training workgroup (64 rows, 4 wavefronts).
+// LDS row strides in BF16: 84 and 36 dwords, so the 16 rows an MFMA operand
+// reads start in different banks.
+constexpr int kXs = 168;  // input rows (>= kMlpIn)
+constexpr int kAs = 72;   // rows of 64: hidden activations, gradients, transposed copies
+constexpr int kDs = 68;   // FP32 gradient rows of 64, in floats
+
+// Shared memory of one training workgroup (64 rows, 16 wavefronts).
 struct TrainSmem {
-    uint16_t x[64 * kMlpIn];      // inputs, row-major
-    uint16_t xt[kMlpIn * 64];     // inputs transposed [k][m]
-    uint16_t a[3][64 * 64];       // hidden activations (post-ReLU), row-major
-    uint16_t at[3][64 * 64];      // transposed
-    float y[64 * 16];             // outputs (fp32, 3 used)
-    float dz[64 * 64];            // current layer's gradient, fp32 [m][n]
-    uint16_t dzb[64 * 64];        // BF16 row-major [m][n]
-    uint16_t dzt[64 * 64];        // BF16 transposed [n][m]
-    float red[4];
+    uint16_t x[64 * kXs];       // inputs, row-major [m][k]
+    uint16_t xt[kMlpIn * kAs];  // inputs transposed [k][m]
+    uint16_t at[3][64 * kAs];   // hidden activations (post-ReLU), transposed [n][m]
+    // two row-major [m][n] buffers in turn: the activations the next layer
+    // reads, then the BF16 gradients the layer below reads
+    uint16_t ab[2][64 * kAs];
+    float dz[2][64 * kDs];       // a layer's gradient, FP32 [m][n] (bias gradients)
+    uint16_t dzt[2][64 * kAs];  // BF16, transposed [n][m] (weight gradients)
+    float err[64 * 4];           // output errors [m][n]
 };
 
-// Writes a 16x16 FP32 tile into LDS as bias + ReLU -> BF16 row-major and
-// transposed activations.
-__device__ __forceinline__ void store_act(f32x4 acc, int m0, int n0, const float *bias, bool relu, uint16_t *a,
-                                         uint16_t *at, int ld) {
+// A K-step's operand fragment of lane l: row r0 + l % 16, columns k0 + 8 (l / 16) .. + 7
+__device__ __forceinline__ bf16x8 mfma_frag(const uint16_t *p, int ld, int r0, int k0) {
     const int lane = threadIdx.x & 63;
-    const int n = n0 + (lane & 15), mb = m0 + (lane >> 4) * 4;
-    for (int i = 0; i < 4; ++i) {
-        float v = acc[i] + bias[n];
-        if (relu) v = v > 0.f ? v : 0.f;
-        const uint16_t h = f2bf(v);
-        a[(mb + i) * ld + n] = h;
-        at[n * 64 + mb + i] = h;
-    }
+    return *(const bf16x8 *)(p + (r0 + (lane & 15)) * ld + k0 + (lane >> 4) * 8);
 }
 
-__global__ __launch_bounds__(256) void k_mlp_train(MlpDev W, const uint16_t *__restrict__ X,
-                                                   const float4 *__restrict__ labels, int npts, int batch,
-                                                   uint32_t seed, int step, float *partials) {
+// Forward and backward of 64 minibatch rows: 16 wavefronts, each one 16x16 tile
+// (rows m0, units n0) of every layer.  What bounds it is the chain of layers:
+// seven dependent products with a barrier and an LDS round trip after each, on
+// matrices too small to fill a CU.  So a layer is one tile per wavefront (2-5
+// MFMAs), every weight fragment, bias and label is in flight before the first
+// barrier, and LDS rows are padded (rows of 64 and 160 BF16 without padding put
+// the 16 rows of an operand into the same banks, and the scattered two-byte
+// transposes of the inputs too).  Batch 4096 (64 workgroups): 31.7 us with four
+// wavefronts and unpadded rows, 14.8 us now.
+// The sums keep their order: MFMA K-steps ascending, bias gradients and the loss
+// by rows.
+__global__ __launch_bounds__(1024) void k_mlp_train(MlpDev W, const uint16_t *__restrict__ X,
+                                                    const float4 *__restrict__ labels, int npts, int batch,
+                                                    uint32_t seed, int step, float *partials) {
     extern __shared__ __align__(16) unsigned char smem_raw[];
     TrainSmem &S = *reinterpret_cast<TrainSmem *>(smem_raw);
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    const int row0 = blockIdx.x * 64;
-    // gather the minibatch rows: row j of the global batch uses sample hash(seed, step, j) % npts
-    for (int i = tid; i < 64 * (kMlpIn / 8); i += 256) {
-        const int m = i / (kMlpIn / 8), c8 = i % (kMlpIn / 8);
-        const uint32_t pick = mix_hash(seed ^ mix_hash((uint32_t)step * 0x9e3779b9u + (uint32_t)(row0 + m))) %
-                              (uint32_t)npts;
-        const uint4 v = *(const uint4 *)(X + (size_t)pick * kMlpIn + c8 * 8);
-        *(uint4 *)(S.x + m * kMlpIn + c8 * 8) = v;
-        const uint16_t *h = (const uint16_t *)&v;
-        for (int j = 0; j < 8; ++j) S.xt[(c8 * 8 + j) * 64 + m] = h[j];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int m0 = (wave & 3) * 16, n0 = (wave >> 2) * 16;
+    const int n = lane & 15, mb = m0 + (lane >> 4) * 4;  // a result tile: rows mb .. mb+3 of column n0 + n
+    // row j of the global batch uses sample hash(seed, step, j) % npts; lane m holds row m's
+    const uint32_t pick = mix_hash(seed ^ mix_hash((uint32_t)step * 0x9e3779b9u + blockIdx.x * 64u + (uint32_t)lane)) %
+                          (uint32_t)npts;
+    // inputs: 20 16-byte chunks of every row, chunk c by wavefront c % 16
+    const uint4 *row = (const uint4 *)(X + (size_t)pick * kMlpIn);
+    const uint4 x0 = row[wave];
+    uint4 x1 = make_uint4(0u, 0u, 0u, 0u);
+    if (wave < 4) x1 = row[16 + wave];
+    // weight fragments, biases and labels
+    bf16x8 w1[5], w2[2], w3[2], w4[2], w4t, w3t[2], w2t[2];
+#pragma unroll
+    for (int k = 0; k < 5; ++k) w1[k] = mfma_frag(W.w1, kMlpIn, n0, k * 32);
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+        w2[k] = mfma_frag(W.w2, 64, n0, k * 32);
+        w3[k] = mfma_frag(W.w3, 64, n0, k * 32);
+        w4[k] = mfma_frag(W.w4, 64, 0, k * 32);
+        w3t[k] = mfma_frag(W.w3t, 64, n0, k * 32);
+        w2t[k] = mfma_frag(W.w2t, 64, n0, k * 32);
     }
-    __syncthreads();
-    // forward: each wavefront computes a 16-row stripe of every layer
-    const int m0 = wave * 16;
-    for (int nt = 0; nt < 4; ++nt) {
-        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-        acc = mfma_tile(S.x, kMlpIn, W.w1, kMlpIn, m0, nt * 16, kMlpIn, acc);
-        store_act(acc, m0, nt * 16, bias_ptr(W.master, 0), true, S.a[0], S.at[0], 64);
+    w4t = mfma_frag(W.w4t, 32, n0, 0);
+    const float b1 = bias_ptr(W.master, 0)[n0 + n], b2 = bias_ptr(W.master, 1)[n0 + n],
+                b3 = bias_ptr(W.master, 2)[n0 + n], b4 = n < 3 ? bias_ptr(W.master, 3)[n] : 0.f;
+    float target[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const uint32_t pk = (uint32_t)__shfl((int)pick, mb + i, 64);
+        target[i] = wave < 4 && n < 3 ? ((const float *)&labels[pk])[n] : 0.f;
     }
-    __syncthreads();
-    for (int nt = 0; nt < 4; ++nt) {
-        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-        acc = mfma_tile(S.a[0], 64, W.w2, 64, m0, nt * 16, 64, acc);
-        store_act(acc, m0, nt * 16, bias_ptr(W.master, 1), true, S.a[1], S.at[1], 64);
-    }
-    __syncthreads();
-    for (int nt = 0; nt < 4; ++nt) {
-        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-        acc = mfma_tile(S.a[1], 64, W.w3, 64, m0, nt * 16, 64, acc);
-        store_act(acc, m0, nt * 16, bias_ptr(W.master, 2), true, S.a[2], S.at[2], 64);
-    }
-    __syncthreads();
     {
-        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-        acc = mfma_tile(S.a[2], 64, W.w4, 64, m0, 0, 64, acc);
-        const int n = lane & 15, mb = m0 + (lane >> 4) * 4;
-        const float *b4 = bias_ptr(W.master, 3);
-        for (int i = 0; i < 4; ++i) S.y[(mb + i) * 16 + n] = acc[i] + (n < 3 ? b4[n] : 0.f);
+        const int c = wave;
+        *(uint4 *)(S.x + lane * kXs + c * 8) = x0;
+        const uint16_t *h = (const uint16_t *)&x0;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) S.xt[(c * 8 + j) * kAs + lane] = h[j];
+    }
+    if (wave < 4) {
+        const int c = 16 + wave;
+        *(uint4 *)(S.x + lane * kXs + c * 8) = x1;
+        const uint16_t *h = (const uint16_t *)&x1;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) S.xt[(c * 8 + j) * kAs + lane] = h[j];
     }
     __syncthreads();
-    // output gradient of the mean squared error over batch x 3 outputs
-    const float inv_n = 2.0f / ((float)batch * 3.0f);
-    float lsum = 0.f;
-    for (int i = tid; i < 64 * 64; i += 256) {
-        const int m = i >> 6, n = i & 63;
-        float d = 0.f;
-        if (n < 3) {
-            const uint32_t pick = mix_hash(seed ^ mix_hash((uint32_t)step * 0x9e3779b9u + (uint32_t)(row0 + m))) %
-                                  (uint32_t)npts;
-            const float4 t = labels[pick];
-            const float tv = (n == 0 ? t.x : (n == 1 ? t.y : t.z)) / W.out_scale;
-            const float e = S.y[m * 16 + n] - tv;
-            lsum += e * e;
-            d = inv_n * e;
+    // forward
+    uint32_t mask[3];  // bit i: this lane's activation of row mb + i is positive
+    auto store_act = [&](f32x4 acc, float bias, int layer, uint16_t *a) {
+        uint32_t h[4];
+        mask[layer] = 0u;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const float v = acc[i] + bias;
+            h[i] = f2bf(v > 0.f ? v : 0.f);
+            mask[layer] |= (h[i] != 0u ? 1u : 0u) << i;
+            a[(mb + i) * kAs + n0 + n] = (uint16_t)h[i];
         }
-        S.dz[i] = d;
-        S.dzb[i] = f2bf(d);
-        S.dzt[n * 64 + m] = S.dzb[i];
+        *(uint2 *)(S.at[layer] + (n0 + n) * kAs + mb) = make_uint2(h[0] | (h[1] << 16), h[2] | (h[3] << 16));
+    };
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int k = 0; k < 5; ++k)
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(mfma_frag(S.x, kXs, m0, k * 32), w1[k], acc, 0, 0, 0);
+    store_act(acc, b1, 0, S.ab[0]);
+    __syncthreads();
+    acc = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int k = 0; k < 2; ++k)
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(mfma_frag(S.ab[0], kAs, m0, k * 32), w2[k], acc, 0, 0, 0);
+    store_act(acc, b2, 1, S.ab[1]);
+    __syncthreads();
+    acc = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int k = 0; k < 2; ++k)
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(mfma_frag(S.ab[1], kAs, m0, k * 32), w3[k], acc, 0, 0, 0);
+    store_act(acc, b3, 2, S.ab[0]);
+    __syncthreads();
+    // outputs and the gradient of the mean squared error over batch x 3 outputs
+    // (unit 16 and up: the zero padding of the 32 units w4t has)
+    auto store_grad = [&](const float g[4], int nn, int cur, uint16_t *b) {
+        uint32_t h[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            h[i] = f2bf(g[i]);
+            S.dz[cur][(mb + i) * kDs + nn] = g[i];
+            b[(mb + i) * kAs + nn] = (uint16_t)h[i];
+        }
+        *(uint2 *)(S.dzt[cur] + nn * kAs + mb) = make_uint2(h[0] | (h[1] << 16), h[2] | (h[3] << 16));
+    };
+    if (wave < 8) {
+        float d[4] = {0.f, 0.f, 0.f, 0.f};
+        if (wave < 4) {
+            const float inv_n = 2.0f / ((float)batch * 3.0f);
+            acc = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int k = 0; k < 2; ++k)
+                acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(mfma_frag(S.ab[0], kAs, m0, k * 32), w4[k], acc, 0, 0, 0);
+            if (n < 3) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const float e = (acc[i] + b4) - target[i] / W.out_scale;
+                    S.err[(mb + i) * 4 + n] = e;
+                    d[i] = inv_n * e;
+                }
+            }
+        }
+        store_grad(d, n0 + n, 0, S.ab[1]);
     }
-    for (int off = 32; off > 0; off >>= 1) lsum += __shfl_xor(lsum, off, 64);
-    if (lane == 0) S.red[wave] = lsum;
     __syncthreads();
     float *P = partials + (size_t)blockIdx.x * kMlpPartialStride;
-    if (tid == 0) P[kMlpParams] = (S.red[0] + S.red[1] + S.red[2] + S.red[3]) / ((float)batch * 3.0f);
-    // backward, layers 4 .. 1.  dW[n][k] = sum_m dz[m][n] a[m][k]: MFMA with
-    // rows n (from dz transposed), columns k (activations transposed), K = m.
-    const int woff[4] = {0, kMlpW1 + 64, kMlpW1 + 64 + kMlpW2 + 64, kMlpW1 + 64 + kMlpW2 + 64 + kMlpW3 + 64};
-    const int fan_in[4] = {129, 64, 64, 64};
-    const int fan_out[4] = {64, 64, 64, 3};
-    for (int layer = 3; layer >= 0; --layer) {
-        const uint16_t *actT = layer == 0 ? S.xt : S.at[layer - 1];
-        const int K_in = layer == 0 ? kMlpIn : 64;
-        const int nrow_tiles = layer == 3 ? 1 : 4;  // output units / 16
-        const int ncol_tiles = K_in / 16;
-        for (int t = wave; t < nrow_tiles * ncol_tiles; t += 4) {
-            const int rt = t / ncol_tiles, ct = t % ncol_tiles;
-            f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-            acc = mfma_tile(S.dzt, 64, actT, 64, rt * 16, ct * 16, 64, acc);
-            const int k = ct * 16 + (lane & 15), nb = rt * 16 + (lane >> 4) * 4;
-            for (int i = 0; i < 4; ++i) {
-                const int n = nb + i;
-                if (n < fan_out[layer] && k < fan_in[layer]) P[woff[layer] + n * fan_in[layer] + k] = acc[i];
+    // dW[n][k] = sum_m dz[m][n] a[m][k]: rows n (dz transposed), columns k
+    // (activations transposed), K = m
+    auto grad_w = [&](const uint16_t *dzt, const uint16_t *at, int rt, int ct, float *out, int fan_in, int fan_out) {
+        f32x4 g = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int k = 0; k < 2; ++k)
+            g = __builtin_amdgcn_mfma_f32_16x16x32_bf16(mfma_frag(dzt, kAs, rt * 16, k * 32),
+                                                        mfma_frag(at, kAs, ct * 16, k * 32), g, 0, 0, 0);
+        const int kk = ct * 16 + n, nb = rt * 16 + (lane >> 4) * 4;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            if (nb + i < fan_out && kk < fan_in) out[(nb + i) * fan_in + kk] = g[i];
+    };
+    // db[n]: the FP32 dz summed over the 64 rows in order
+    auto grad_b = [&](const float *dz, float *out, int fan_out) {
+        if (lane >= fan_out) return;
+        float s = 0.f;
+#pragma unroll 16
+        for (int m = 0; m < 64; ++m) s += dz[m * kDs + lane];
+        out[lane] = s;
+    };
+    constexpr int o1 = 0, o2 = kMlpW1 + 64, o3 = o2 + kMlpW2 + 64, o4 = o3 + kMlpW3 + 64;
+    float g[4];
+    // layer 4 (dz 0, rows in ab[1]) -> the gradient of layer 3's units (dz 1, ab[0])
+    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(mfma_frag(S.ab[1], kAs, m0, 0), w4t, f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) g[i] = (mask[2] >> i) & 1u ? acc[i] : 0.f;
+    store_grad(g, n0 + n, 1, S.ab[0]);
+    if (wave < 4) grad_w(S.dzt[0], S.at[2], 0, wave, P + o4, 64, 3);
+    if (wave == 4) grad_b(S.dz[0], P + o4 + kMlpW4, 3);
+    if (wave == 5) {
+        // the loss: output n of rows w, w + 4, ... in order (lane 3 w + n), then
+        // (n0 + n2) + n1 of each w, then the four w in order
+        float l = 0.f;
+        const int w = lane / 3, nn = lane % 3;
+        if (lane < 12) {
+#pragma unroll
+            for (int j = 0; j < 16; ++j) {
+                const float e = S.err[(w + 4 * j) * 4 + nn];
+                l += e * e;
             }
         }
-        // bias gradient: sum over the 64 rows of the fp32 dz
-        for (int n = tid; n < fan_out[layer]; n += 256) {
-            float s = 0.f;
-            for (int m = 0; m < 64; ++m) s += S.dz[m * 64 + n];
-            P[woff[layer] + fan_out[layer] * fan_in[layer] + n] = s;
+        float t = 0.f;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const float q = (__shfl(l, 3 * k, 64) + __shfl(l, 3 * k + 2, 64)) + __shfl(l, 3 * k + 1, 64);
+            t = k == 0 ? q : t + q;
         }
-        if (layer == 0) break;
-        __syncthreads();
-        // da[m][k] = sum_n dz[m][n] W[n][k]: rows m (dz row-major), columns k
-        // (W transposed, [k][n]); then dz_prev = da * (a > 0)
-        const uint16_t *wt = layer == 3 ? W.w4t : (layer == 2 ? W.w3t : W.w2t);
-        const int Kn = layer == 3 ? 32 : 64;
-        f32x4 da[4];
-        for (int ct = 0; ct < 4; ++ct) {
-            f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-            da[ct] = mfma_tile(S.dzb, 64, wt, Kn, m0, ct * 16, Kn, acc);
-        }
-        __syncthreads();  // everyone has read dzb before it is overwritten
-        const uint16_t *aprev = S.a[layer - 1];
-        for (int ct = 0; ct < 4; ++ct) {
-            const int n = ct * 16 + (lane & 15), mb = m0 + (lane >> 4) * 4;
-            for (int i = 0; i < 4; ++i) {
-                const int m = mb + i;
-                const float g = bf2f(aprev[m * 64 + n]) > 0.f ? da[ct][i] : 0.f;
-                S.dz[m * 64 + n] = g;
-                const uint16_t h = f2bf(g);
-                S.dzb[m * 64 + n] = h;
-                S.dzt[n * 64 + m] = h;
-            }
-        }
-        __syncthreads();
+        if (lane == 0) P[kMlpParams] = t / ((float)batch * 3.0f);
     }
+    __syncthreads();
+    // layer 3 (dz 1, ab[0]) -> layer 2's units (dz 0, ab[1])
+    acc = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int k = 0; k < 2; ++k)
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(mfma_frag(S.ab[0], kAs, m0, k * 32), w3t[k], acc, 0, 0, 0);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) g[i] = (mask[1] >> i) & 1u ? acc[i] : 0.f;
+    store_grad(g, n0 + n, 0, S.ab[1]);
+    grad_w(S.dzt[1], S.at[1], wave & 3, wave >> 2, P + o3, 64, 64);
+    if (wave == 0) grad_b(S.dz[1], P + o3 + kMlpW3, 64);
+    __syncthreads();
+    // layer 2 (dz 0, ab[1]) -> layer 1's units (dz 1, ab[0])
+    acc = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int k = 0; k < 2; ++k)
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(mfma_frag(S.ab[1], kAs, m0, k * 32), w2t[k], acc, 0, 0, 0);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) g[i] = (mask[0] >> i) & 1u ? acc[i] : 0.f;
+    store_grad(g, n0 + n, 1, S.ab[0]);
+    grad_w(S.dzt[0], S.at[0], wave & 3, wave >> 2, P + o2, 64, 64);
+    if (wave == 0) grad_b(S.dz[0], P + o2 + kMlpW2, 64);
+    __syncthreads();
+    // layer 1: 4 x 9 tiles (the tenth column tile is padding)
+    for (int t = wave; t < 36; t += 16) grad_w(S.dzt[1], S.xt, t & 3, t >> 2, P + o1, 129, 64);
+    if (wave == 15) grad_b(S.dz[1], P + o1 + kMlpW1, 64);
 }
 
 // Sums the per-workgroup partial gradients and applies Adam to the FP32
 // master weights; re-emits the BF16 operand copies.
-__global__ __launch_bounds__(256) void k_adam(float *master, float *m1, float *m2, const float *partials,
-                                              int nparts, float lr, float b1, float b2, float eps, int step,
-                                              uint16_t *w1, uint16_t *w2, uint16_t *w3, uint16_t *w4, uint16_t *w2t,
-                                              uint16_t *w3t, uint16_t *w4t, float *loss_out) {
+//
+// Bound by the latency of the partials, which another XCD's L2 has just
+// written back: one wavefront per workgroup spreads the parameters over all
+// CUs, and 16 loads of a parameter's partials are in flight at a time (they
+// are added in workgroup order).  Batch 4096: 21.3 us with 256-thread
+// workgroups, 5.2 us now.
+__global__ __launch_bounds__(64) void k_adam(float *master, float *m1, float *m2, const float *__restrict__ partials,
+                                             int nparts, float lr, float b1, float b2, float eps, int step,
+                                             uint16_t *w1, uint16_t *w2, uint16_t *w3, uint16_t *w4, uint16_t *w2t,
+                                             uint16_t *w3t, uint16_t *w4t, float *loss_out) {
     const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p == kMlpParams && loss_out) {
-        float l = 0.f;
-        for (int i = 0; i < nparts; ++i) l += partials[(size_t)i * kMlpPartialStride + kMlpParams];
-        loss_out[0] = l;
-    }
-    if (p >= kMlpParams) return;
+    if (p > kMlpParams) return;
     float g = 0.f;
-    for (int i = 0; i < nparts; ++i) g += partials[(size_t)i * kMlpPartialStride + p];
+    int i = 0;
+    for (; i + 16 <= nparts; i += 16) {
+        float q[16];
+#pragma unroll
+        for (int k = 0; k < 16; ++k) q[k] = partials[(size_t)(i + k) * kMlpPartialStride + p];
+#pragma unroll
+        for (int k = 0; k < 16; ++k) g += q[k];
+    }
+    for (; i < nparts; ++i) g += partials[(size_t)i * kMlpPartialStride + p];
+    if (p == kMlpParams) {  // the loss, after the parameters' gradients
+        if (loss_out) loss_out[0] = g;
+        return;
+    }
     const float m = b1 * m1[p] + (1.f - b1) * g;
     const float v = b2 * m2[p] + (1.f - b2) * g * g;
     m1[p] = m;
@@ -662,9 +738,6 @@ __global__ __launch_bounds__(256) void k_adam(float *master, float *m1, float *m
 // the B operand, so a lane's four results are four consecutive units of one
 // pixel and leave as one 8-byte LDS store.  Row strides of 168 and 72 BF16 (84
 // and 36 dwords) make a tile's 16 row reads hit disjoint LDS banks.
-constexpr int kXs = 168;  // input row stride (>= kMlpIn)
-constexpr int kAs = 72;   // hidden activation row stride (>= 64)
-
 struct InferSmem {
     uint16_t x[64 * kXs];  // inputs, then hidden activations (stride kAs)
     float y[64 * 4];
@@ -1090,11 +1163,11 @@ hipError_t launch_mlp_train_step(MlpBuffers &B, const uint16_t *X, const float4 
         if (e != hipSuccess) return e;
         smem_attr = true;
     }
-    hipLaunchKernelGGL(k_mlp_train, dim3(nblk), dim3(256), sizeof(TrainSmem), s, mlp_dev(B), X, labels, npts, batch,
+    hipLaunchKernelGGL(k_mlp_train, dim3(nblk), dim3(1024), sizeof(TrainSmem), s, mlp_dev(B), X, labels, npts, batch,
                        seed, step, B.partials);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(k_adam, dim3((kMlpParams + 1 + 255) / 256), dim3(256), 0, s, B.master, B.m1, B.m2, B.partials,
+    hipLaunchKernelGGL(k_adam, dim3((kMlpParams + 1 + 63) / 64), dim3(64), 0, s, B.master, B.m1, B.m2, B.partials,
                        nblk, lr, b1, b2, eps, step, B.w1, B.w2, B.w3, B.w4, B.w2t, B.w3t, B.w4t, loss_out);
     return hipGetLastError();
 }
