@@ -386,7 +386,7 @@ int vct_create(vct_ctx **out, const vct_grid_desc *desc) {
     }
     if (hipMalloc((void **)&c->d_partials, kStatPartials * 4 * sizeof(uint32_t)) != hipSuccess ||
         hipMalloc((void **)&c->d_stats, sizeof(vct_stats)) != hipSuccess ||
-        hipMemset(c->d_stats, 0, sizeof(vct_stats)) != hipSuccess) {
+        hipMemsetAsync(c->d_stats, 0, sizeof(vct_stats), c->stream) != hipSuccess) {
         vct_destroy(c);
         return fail(nullptr, VCT_ERR_NOMEM, "stats allocation failed");
     }
@@ -1048,10 +1048,12 @@ static int ensure_camera(vct_ctx *c, int w, int h) {
     HIPCHK(c, dalloc(&c->d_ind, np * 16));
     HIPCHK(c, dalloc(&c->d_spec, np * 16));
     HIPCHK(c, dalloc(&c->d_color, np * 16));
-    HIPCHK(c, hipMemset(c->d_color, 0, np * 16));
-    HIPCHK(c, hipMemset(c->d_gbuf, 0, np * sizeof(vct_gbuffer_texel)));
-    HIPCHK(c, hipMemset(c->d_ind, 0, np * 16));
-    HIPCHK(c, hipMemset(c->d_spec, 0, np * 16));
+    // on the context's stream: a null-stream clear may still be running when the
+    // call returns, and nothing orders it before the passes
+    HIPCHK(c, hipMemsetAsync(c->d_color, 0, np * 16, c->stream));
+    HIPCHK(c, hipMemsetAsync(c->d_gbuf, 0, np * sizeof(vct_gbuffer_texel), c->stream));
+    HIPCHK(c, hipMemsetAsync(c->d_ind, 0, np * 16, c->stream));
+    HIPCHK(c, hipMemsetAsync(c->d_spec, 0, np * 16, c->stream));
     c->gw = w;
     c->gh = h;
     c->have_gbuf = false;
@@ -1362,10 +1364,11 @@ static int ensure_mlp(vct_ctx *c) {
     HIPCHK(c, dalloc(&B.w2t, 64 * 64 * 2));
     HIPCHK(c, dalloc(&B.w3t, 64 * 64 * 2));
     HIPCHK(c, dalloc(&B.w4t, 64 * 32 * 2));
-    HIPCHK(c, hipMemset(B.w1, 0, (size_t)64 * kMlpIn * 2));
-    HIPCHK(c, hipMemset(B.w4, 0, 16 * 64 * 2));
-    HIPCHK(c, hipMemset(B.w4t, 0, 64 * 32 * 2));
-    HIPCHK(c, hipMemset(B.master, 0, (size_t)kMlpParams * 4));
+    // on the context's stream, before whatever is copied over them
+    HIPCHK(c, hipMemsetAsync(B.w1, 0, (size_t)64 * kMlpIn * 2, c->stream));
+    HIPCHK(c, hipMemsetAsync(B.w4, 0, 16 * 64 * 2, c->stream));
+    HIPCHK(c, hipMemsetAsync(B.w4t, 0, 64 * 32 * 2, c->stream));
+    HIPCHK(c, hipMemsetAsync(B.master, 0, (size_t)kMlpParams * 4, c->stream));
     return VCT_OK;
 }
 
@@ -1453,9 +1456,10 @@ int vct_learned_train(vct_ctx *c, const vct_learned_params *p, float *loss) {
             for (int i = 0; i < fin[l] * fout[l]; ++i) w[o++] = (float)U(rng);
             o += fout[l];
         }
-        HIPCHK(c, hipMemcpy(B.master, w.data(), (size_t)kMlpParams * 4, hipMemcpyHostToDevice));
-        HIPCHK(c, hipMemset(B.m1, 0, (size_t)kMlpParams * 4));
-        HIPCHK(c, hipMemset(B.m2, 0, (size_t)kMlpParams * 4));
+        HIPCHK(c, hipMemcpyAsync(B.master, w.data(), (size_t)kMlpParams * 4, hipMemcpyHostToDevice, c->stream));
+        HIPCHK(c, hipMemsetAsync(B.m1, 0, (size_t)kMlpParams * 4, c->stream));
+        HIPCHK(c, hipMemsetAsync(B.m2, 0, (size_t)kMlpParams * 4, c->stream));
+        HIPCHK(c, hipStreamSynchronize(c->stream));  // the copy reads w
         LAUNCHCHK(c, launch_emit_operands(B, c->stream));
         c->have_weights = true;
         c->adam_t = 0;
