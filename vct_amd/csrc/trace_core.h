@@ -29,12 +29,24 @@ namespace vctk {
 // hold one 16-byte texel per element: eight loads.
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
+// What the sampler needs of a level, by value in the kernel arguments: a level
+// index is wave-uniform, so its fields are scalar loads whatever the kernel has
+// stored before (behind a pointer the compiler has to load them per lane after
+// the first store, and every product with them becomes vector work).
+struct SampleLevel {
+    float fs;             // edge length
+    uint32_t org;         // byte offset of the level's storage (its first border brick)
+    uint32_t sx, sy, sz;  // LevelInfo strides
+    int nfaces;
+    int one;              // one fp32 texel per element instead of an fp16 pair
+    int pad;
+};
 struct PyrArgs {
     const char *pyr;
     uint32_t bytes;
-    const LevelInfo *lv;
     int dim, nlevels;
     int nested;  // TraceLaunch::nested
+    SampleLevel lv[VCT_MAX_LEVELS];
 };
 
 __device__ __forceinline__ uint4 bload16(__amdgpu_buffer_rsrc_t r, uint32_t off) {
@@ -91,9 +103,9 @@ __device__ __forceinline__ void warp_sample_march(const float4 *__restrict__ wm,
     for (int k = 0; k < 3; ++k) p[k] = acc[k];
 }
 
-// All 2x2x2 texels of a uniform fetch are +0 (empty space): their weighted sum
-// adds exactly 0, so the weighting is skipped.  The test runs on the scalar
-// unit, beside the vector work of the other wavefronts.
+// All texels of a uniform fetch are +0 (empty space): their weighted sum adds
+// exactly 0, so the weighting is skipped.  The test runs on the scalar unit,
+// beside the vector work of the other wavefronts.
 template <int N>
 __device__ __forceinline__ bool zero16(const uint4 (&v)[N]) {
     uint32_t o = 0u;
@@ -102,21 +114,8 @@ __device__ __forceinline__ bool zero16(const uint4 (&v)[N]) {
     return o == 0u;
 }
 
-// The sampler's axis terms: the border bricks hold texels -1 and s as zeros,
-// so neither index is clamped nor weight masked.  Indices are shifted by one
-// brick (+4, never negative for the 24-bit multiplies; brick index < 2^7 + 2,
-// stride < 2^24 for dim <= 512) and offsets are taken from the level's storage
-// start.
-__device__ __forceinline__ void axis_terms_pad(float p, int s, uint32_t mul, uint32_t sub, uint32_t t[2], float w[2]) {
-    const float u = p * (float)s - 0.5f;
-    const float fl = __builtin_floorf(u);
-    const int i0 = (int)fl + 4;  // texel -1 .. s-1, shifted
-    const float f = u - fl;
-    w[0] = 1.0f - f;
-    w[1] = f;
-    t[0] = __umul24((uint32_t)(i0 >> 2), mul) + (uint32_t)(i0 & 3) * sub;
-    // texel i0 + 1: the next one in the brick, or the first of the next brick
-    t[1] = t[0] + ((i0 & 3) == 3 ? mul - 3u * sub : sub);
+__device__ __forceinline__ uint64_t or16(const uint4 &v) {
+    return ((uint64_t)v.y << 32 | v.x) | ((uint64_t)v.w << 32 | v.z);
 }
 
 __device__ __forceinline__ float hlo(uint32_t v) { return __half2float(__ushort_as_half((uint16_t)(v & 0xffffu))); }
@@ -140,200 +139,221 @@ __device__ __forceinline__ void acc_f4(float4 &acc, uint4 v, float w) {
     acc.z = fmaf(__uint_as_float(v.z), w, acc.z);
     acc.w = fmaf(__uint_as_float(v.w), w, acc.w);
 }
+__device__ __forceinline__ void acc_face(float4 &acc, const float4 &t, float d2) {
+    acc.x = fmaf(t.x, d2, acc.x);
+    acc.y = fmaf(t.y, d2, acc.y);
+    acc.z = fmaf(t.z, d2, acc.z);
+    acc.w = fmaf(t.w, d2, acc.w);
+}
+// Keeps the scalar path's arithmetic out of the per-lane path's: the two end
+// alike, and merged they would move every texel through vector registers.
+__device__ __forceinline__ void keep_apart(float4 &acc) {
+    asm volatile("" : "+v"(acc.x), "+v"(acc.y), "+v"(acc.z), "+v"(acc.w));
+}
 
-// acc += lw * (trilinear sample of level L at p), for levels of one 16-byte
-// fp32 texel per element (fp32 storage; the decoded copy of an fp8 level).  The
-// arguments and the wave-uniform scalar path are those of level_sample below.
-// The offsets of the eight corners are sums of the axis terms, formed as they
-// are used.  Bound by VALU issue in the scalar path (40 instructions per face)
-// and by the texture-address unit in the per-lane one (eight loads per face).
-// Measured: the FP8 trace of the 3840x2160 warped scene 28.9 -> 9 ms and of a
-// 961x541 frame 1.72 -> 0.55 ms against four-byte loads decoded per corner
-// (their decoder made the sampler a called function with scratch memory); the
-// isotropic FP32 gather at 1001x567 242 -> 223 us.  Texels are weighted and
-// summed in one fixed order (w[k] * d2 into acc): a march compares its opacity
-// with 0.95, and sums that differ in the last bit end some cones a step apart.
-template <bool ZQ>
-__device__ __forceinline__ bool level_sample_f32(float4 &acc, const char *pyr, __amdgpu_buffer_rsrc_t rs,
-                                                 const LevelInfo &L, const float p[3], float lw, const uint32_t fe[3],
-                                                 const float d2[3], uint32_t fmask, bool fsame) {
-    const int s = L.size;
+// The faces of a cone's direction: byte offsets of the three that face it, per
+// lane and of the first lane, their weights dir^2, fmask (wave-uniform: bit a
+// set unless weight a is 0 in every lane) and whether every lane has the first
+// lane's faces.
+struct ConeFaces {
+    uint32_t fe[3], sfe[3];
+    float d2[3];
+    uint32_t fmask;
+    bool fsame;
+};
+
+// The element offsets of texels i and i + 1 along an axis (i shifted by the
+// border brick): the next one in the brick, or the first of the next brick.
+// Brick index < 2^8, stride < 2^24 (dim <= 512): full-rate 24-bit multiplies.
+__device__ __forceinline__ void axis_terms(uint32_t i, uint32_t mul, uint32_t sub, uint32_t t[2]) {
+    t[0] = __umul24(i >> 2, mul) + (i & 3u) * sub;
+    t[1] = t[0] + ((i & 3u) == 3u ? mul - 3u * sub : sub);
+}
+
+// The same of a wave-uniform index on the scalar unit, which has no 24-bit
+// multiply (__umul24 would move the address, and the loads, to the vector side).
+__device__ __forceinline__ void axis_terms_s(uint32_t i, uint32_t mul, uint32_t sub, uint32_t t[2]) {
+    t[0] = (i >> 2) * mul + (i & 3u) * sub;
+    t[1] = t[0] + ((i & 3u) == 3u ? mul - 3u * sub : sub);
+}
+
+// acc += lw * (trilinear sample of level l at p): isotropic, or the
+// dir^2-weighted mix of the three faces that face the cone.  l is wave-uniform.
+// The border bricks hold texels -1 and s as zeros, so no index is clamped and
+// no weight masked; indices are shifted by one brick (+4).  Returns
+// (wave-uniform) whether every texel fetched, in every lane, was +0 (ZQ: also
+// test the per-lane fetches, which costs vector instructions).  An fp8 level
+// reports false: its codes underflow, so a zero there does not say that the
+// finer level is zero.
+//
+// At 1080p a wavefront's 8x8 pixels span about a voxel, so at the coarser
+// levels all its lanes usually need the same 2x2x2 texels (and faces).  They
+// are then fetched once for the wavefront with scalar loads and every lane
+// weights them itself: the same operations on the same values as the per-lane
+// path, without its vector memory traffic.  Whether they do is decided on the
+// packed cell indices, before any address exists: the addresses of a shared
+// cell are scalar arithmetic, and its weights are formed only if one of the
+// cell's texels is not zero.  What bounds the trace is VALU issue (95% of the
+// cycles at 1080p): an empty shared cell costs 12 vector instructions (60 when
+// addresses and weights were formed first), an occupied one 32 plus 36 a face.
+// Texels are weighted and summed in one fixed order: a march compares its
+// opacity with 0.95, and sums that differ in the last bit end some cones a step
+// apart.
+template <int MODE, bool ZQ>
+__device__ __forceinline__ bool level_sample(float4 &acc, const PyrArgs &pa, __amdgpu_buffer_rsrc_t rs, int l,
+                                             const float p[3], float lw, const ConeFaces &cf) {
+    const SampleLevel &L = pa.lv[l];
     const bool aniso = L.nfaces == 6;
-    uint32_t tx[2], ty[2], tz[2];
-    float wx[2], wy[2], wz[2];
-    axis_terms_pad(p[0], s, L.sx, 1u, tx, wx);
-    axis_terms_pad(p[1], s, L.sy, 4u, ty, wy);
-    axis_terms_pad(p[2], s, L.sz, 16u, tz, wz);
-    const uint32_t org = L.stage - L.pad * 16u;  // the level's storage start
-    wz[0] *= lw;
-    wz[1] *= lw;
-    float w[8];
-    uint32_t oyz[4];
+    const bool one = MODE == 1 || (MODE == 2 && L.one);
+    const bool zq = MODE == 1 ? ZQ : (MODE == 2 && L.one ? false : ZQ);  // may a zero be reported
+    float f[3];
+    uint32_t i[3];
 #pragma unroll
-    for (int c = 0; c < 4; ++c) {
-        w[2 * c] = (wx[0] * wy[c & 1]) * wz[c >> 1];
-        w[2 * c + 1] = (wx[1] * wy[c & 1]) * wz[c >> 1];
-        oyz[c] = org + (ty[c & 1] + tz[c >> 1]) * 16u;
+    for (int k = 0; k < 3; ++k) {
+        const float u = p[k] * L.fs - 0.5f;
+        const float fl = __builtin_floorf(u);
+        i[k] = (uint32_t)((int)fl + 4);
+        f[k] = u - fl;
     }
-    const uint32_t o0 = oyz[0] + tx[0] * 16u, o7 = oyz[3] + tx[1] * 16u;
-    const bool same = (!aniso || fsame) && __builtin_amdgcn_readfirstlane(o0) == o0 &&
-                      __builtin_amdgcn_readfirstlane(o7) == o7;
-    const int nf = aniso ? 3 : 1;
-    if (__ballot(same) == __ballot(true)) {
-        const uint32_t sx0 = __builtin_amdgcn_readfirstlane(tx[0]) * 16u, sx1 = __builtin_amdgcn_readfirstlane(tx[1]) * 16u;
-        uint32_t so[4];
+    const uint32_t key = i[0] | (i[1] << 10) | (i[2] << 20);
+    const uint32_t k0 = __builtin_amdgcn_readfirstlane(key);
+    if ((!aniso | cf.fsame) & (__ballot(key != k0) == 0)) {
+        uint32_t tx[2], ty[2], tz[2], so[4];
+        axis_terms_s(k0 & 1023u, L.sx, 1u, tx);
+        axis_terms_s((k0 >> 10) & 1023u, L.sy, 4u, ty);
+        axis_terms_s(k0 >> 20, L.sz, 16u, tz);
 #pragma unroll
-        for (int c = 0; c < 4; ++c) so[c] = __builtin_amdgcn_readfirstlane(oyz[c]);
+        for (int c = 0; c < 4; ++c) so[c] = L.org + (tx[0] + ty[c & 1] + tz[c >> 1]) * 16u;
+        if (one) {
+            const uint32_t dx = (tx[1] - tx[0]) * 16u;
+            bool z = true;
+            float w[8];
+#pragma unroll
+            for (int a = 0; a < 3; ++a) {
+                if (aniso ? !((cf.fmask >> a) & 1u) : a > 0) continue;
+                const uint32_t fo = aniso ? cf.sfe[a] : 0u;
+                uint4 v[8];
+#pragma unroll
+                for (int c = 0; c < 4; ++c) {
+                    v[2 * c] = sload16(pa.pyr, so[c] + fo);
+                    v[2 * c + 1] = sload16(pa.pyr, so[c] + dx + fo);
+                }
+                if (zero16(v)) continue;
+                if (z) {
+                    const float wy[2] = {1.0f - f[1], f[1]}, wz[2] = {(1.0f - f[2]) * lw, f[2] * lw};
+#pragma unroll
+                    for (int c = 0; c < 4; ++c) {
+                        w[2 * c] = ((1.0f - f[0]) * wy[c & 1]) * wz[c >> 1];
+                        w[2 * c + 1] = (f[0] * wy[c & 1]) * wz[c >> 1];
+                    }
+                    z = false;
+                }
+                const float fw = aniso ? cf.d2[a] : 1.0f;
+#pragma unroll
+                for (int k = 0; k < 8; ++k) acc_f4(acc, v[k], w[k] * fw);
+            }
+            keep_apart(acc);
+            return z && (MODE == 1 || !L.one);
+        }
         bool z = true;
-        for (int a = 0; a < nf; ++a) {
-            if (aniso && !((fmask >> a) & 1u)) continue;
-            const uint32_t fo = aniso ? __builtin_amdgcn_readfirstlane(fe[a]) * 16u : 0u;
+        float wa[4], wb[4];
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+            if (aniso ? !((cf.fmask >> a) & 1u) : a > 0) continue;
+            uint4 v[4];
+#pragma unroll
+            for (int c = 0; c < 4; ++c) v[c] = sload16(pa.pyr, so[c] + (aniso ? cf.sfe[a] : 0u));
+            const uint64_t e0 = or16(v[0]), e1 = or16(v[1]), e2 = or16(v[2]), e3 = or16(v[3]);
+            if (((e0 | e1) | (e2 | e3)) == 0) continue;
+            if (z) {
+                const float wy[2] = {1.0f - f[1], f[1]}, wz[2] = {(1.0f - f[2]) * lw, f[2] * lw};
+#pragma unroll
+                for (int c = 0; c < 4; ++c) {
+                    const float wyz = wy[c & 1] * wz[c >> 1];
+                    wa[c] = (1.0f - f[0]) * wyz;
+                    wb[c] = f[0] * wyz;
+                }
+                z = false;
+            }
+            float4 t = aniso ? make_float4(0.f, 0.f, 0.f, 0.f) : acc;
+            if (e0) acc_pair(t, v[0], wa[0], wb[0]);
+            if (e1) acc_pair(t, v[1], wa[1], wb[1]);
+            if (e2) acc_pair(t, v[2], wa[2], wb[2]);
+            if (e3) acc_pair(t, v[3], wa[3], wb[3]);
+            if (!aniso) {
+                acc = t;
+                break;
+            }
+            acc_face(acc, t, cf.d2[a]);
+        }
+        keep_apart(acc);
+        return z;
+    }
+    uint32_t tx[2], ty[2], tz[2], off[4];
+    axis_terms(i[0], L.sx, 1u, tx);
+    axis_terms(i[1], L.sy, 4u, ty);
+    axis_terms(i[2], L.sz, 16u, tz);
+#pragma unroll
+    for (int c = 0; c < 4; ++c) off[c] = L.org + (tx[0] + ty[c & 1] + tz[c >> 1]) * 16u;
+    const float wy[2] = {1.0f - f[1], f[1]}, wz[2] = {(1.0f - f[2]) * lw, f[2] * lw};
+    bool z = zq;
+    if (one) {
+        const uint32_t dx = (tx[1] - tx[0]) * 16u;
+        float w[8];
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            w[2 * c] = ((1.0f - f[0]) * wy[c & 1]) * wz[c >> 1];
+            w[2 * c + 1] = (f[0] * wy[c & 1]) * wz[c >> 1];
+        }
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+            if (aniso ? !((cf.fmask >> a) & 1u) : a > 0) continue;
+            const uint32_t fo = aniso ? cf.fe[a] : 0u;
             uint4 v[8];
 #pragma unroll
             for (int c = 0; c < 4; ++c) {
-                v[2 * c] = sload16(pyr, so[c] + sx0 + fo);
-                v[2 * c + 1] = sload16(pyr, so[c] + sx1 + fo);
+                v[2 * c] = bload16(rs, off[c] + fo);
+                v[2 * c + 1] = bload16(rs, off[c] + dx + fo);
             }
-            if (zero16(v)) continue;
+            if (zq && __ballot(!zero16(v)) == 0) continue;
             z = false;
-            const float fw = aniso ? d2[a] : 1.0f;
+            const float fw = aniso ? cf.d2[a] : 1.0f;
 #pragma unroll
             for (int k = 0; k < 8; ++k) acc_f4(acc, v[k], w[k] * fw);
         }
         return z;
     }
-    bool z = ZQ;
-    for (int a = 0; a < nf; ++a) {
-        if (aniso && !((fmask >> a) & 1u)) continue;
-        const uint32_t fo = aniso ? fe[a] * 16u : 0u;
-        uint4 v[8];
+    float wa[4], wb[4];
+    {
+        const float wlo = 1.0f - f[0], whi = f[0];
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
-            v[2 * c] = bload16(rs, oyz[c] + tx[0] * 16u + fo);
-            v[2 * c + 1] = bload16(rs, oyz[c] + tx[1] * 16u + fo);
+            const float wyz = wy[c & 1] * wz[c >> 1];
+            wa[c] = wlo * wyz;
+            wb[c] = whi * wyz;
         }
-        if (ZQ && __ballot(!zero16(v)) == 0) continue;
-        z = false;
-        const float fw = aniso ? d2[a] : 1.0f;
-#pragma unroll
-        for (int k = 0; k < 8; ++k) acc_f4(acc, v[k], w[k] * fw);
-    }
-    return z;
-}
-
-// acc += lw * (trilinear sample of level L at p): isotropic, or the
-// dir^2-weighted mix of the three faces that face the cone (fe: their element
-// offsets, 64 * face).  L is wave-uniform.  fmask (wave-uniform) has bit a
-// set unless d2[a] is 0 in every lane: a face no lane weights adds exactly 0
-// and is not fetched.  Returns (wave-uniform) whether every texel fetched, in
-// every lane, was +0 (ZQ: also test the per-lane fetches, which costs vector
-// instructions).  An fp8 level reports false: its codes underflow, so a zero
-// there does not say that the finer level is zero.
-template <int MODE, bool ZQ>
-__device__ __forceinline__ bool level_sample(float4 &acc, const char *pyr, __amdgpu_buffer_rsrc_t rs,
-                                             const LevelInfo &L, const float p[3], float lw, const uint32_t fe[3],
-                                             const float d2[3], uint32_t fmask, bool fsame) {
-    if (MODE == 1) return level_sample_f32<ZQ>(acc, pyr, rs, L, p, lw, fe, d2, fmask, fsame);
-    if (MODE == 2 && L.fmt == 2) {
-        level_sample_f32<false>(acc, pyr, rs, L, p, lw, fe, d2, fmask, fsame);
-        return false;
-    }
-    const int s = L.size;
-    const bool aniso = L.nfaces == 6;
-    uint32_t ty[2], tz[2];
-    float wy[2], wz[2];
-    // fp16 pairs: element x holds texels x and x+1, so one load per (y, z)
-    // corner pair; element -1 (border brick) holds (0, texel 0)
-    axis_terms_pad(p[1], s, L.sy, 4u, ty, wy);
-    axis_terms_pad(p[2], s, L.sz, 16u, tz, wz);
-    wz[0] *= lw;
-    wz[1] *= lw;
-    const float u = p[0] * (float)s - 0.5f;
-    const float fl = __builtin_floorf(u);
-    const int cx = (int)fl + 4;  // pair element of texel -1 .. s-1, shifted one brick
-    const float f = u - fl;
-    const float wlo = 1.0f - f, whi = f;
-    const uint32_t ex = __umul24((uint32_t)(cx >> 2), L.sx) + (uint32_t)(cx & 3);
-    const uint32_t org = L.base - L.pad * 16u;  // the level's storage start
-    uint32_t off[4];
-    float wa[4], wb[4];
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {
-        const int dy = c & 1, dz = c >> 1;
-        off[c] = org + (ex + ty[dy] + tz[dz]) * 16u;
-        const float wyz = wy[dy] * wz[dz];
-        wa[c] = wlo * wyz;
-        wb[c] = whi * wyz;
-    }
-    // At 1080p a wavefront's 8x8 pixels span about a voxel, so at the coarser
-    // levels all its lanes usually need the same 2x2x2 texels (and faces).  The
-    // four corner elements are then fetched once for the wavefront with scalar
-    // loads and every lane weights them itself: the same operations on the same
-    // values as the per-lane path, without its vector memory traffic.  Corners
-    // 0 and 3 together fix all four (the element encoding of a texel index is
-    // unique, and corner 3 carries the clamped upper indices).  fsame: the
-    // faces of every lane's cone are the first lane's (wave-uniform, decided
-    // once per cone).
-    const bool same = (!aniso || fsame) && __builtin_amdgcn_readfirstlane(off[0]) == off[0] &&
-                      __builtin_amdgcn_readfirstlane(off[3]) == off[3];
-    if (__ballot(same) == __ballot(true)) {
-        uint32_t so[4];
-#pragma unroll
-        for (int c = 0; c < 4; ++c) so[c] = __builtin_amdgcn_readfirstlane(off[c]);
-        if (!aniso) {
-            uint4 v[4];
-#pragma unroll
-            for (int c = 0; c < 4; ++c) v[c] = sload16(pyr, so[c]);
-            if (zero16(v)) return true;
-#pragma unroll
-            for (int c = 0; c < 4; ++c) acc_pair(acc, v[c], wa[c], wb[c]);
-            return false;
-        }
-        bool z = true;
-#pragma unroll
-        for (int a = 0; a < 3; ++a) {
-            if (!((fmask >> a) & 1u)) continue;
-            const uint32_t fo = __builtin_amdgcn_readfirstlane(fe[a]) * 16u;
-            uint4 v[4];
-#pragma unroll
-            for (int c = 0; c < 4; ++c) v[c] = sload16(pyr, so[c] + fo);
-            if (zero16(v)) continue;
-            z = false;
-            float4 t = make_float4(0.f, 0.f, 0.f, 0.f);
-#pragma unroll
-            for (int c = 0; c < 4; ++c) acc_pair(t, v[c], wa[c], wb[c]);
-            acc.x = fmaf(t.x, d2[a], acc.x);
-            acc.y = fmaf(t.y, d2[a], acc.y);
-            acc.z = fmaf(t.z, d2[a], acc.z);
-            acc.w = fmaf(t.w, d2[a], acc.w);
-        }
-        return z;
     }
     if (!aniso) {
         uint4 v[4];
 #pragma unroll
         for (int c = 0; c < 4; ++c) v[c] = bload16(rs, off[c]);
-        if (ZQ && __ballot(!zero16(v)) == 0) return true;
+        if (zq && __ballot(!zero16(v)) == 0) return true;
 #pragma unroll
         for (int c = 0; c < 4; ++c) acc_pair(acc, v[c], wa[c], wb[c]);
         return false;
     }
-    bool z = ZQ;
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
-        if (!((fmask >> a) & 1u)) continue;
+        if (!((cf.fmask >> a) & 1u)) continue;
         uint4 v[4];
 #pragma unroll
-        for (int c = 0; c < 4; ++c) v[c] = bload16(rs, off[c] + fe[a] * 16u);
-        if (ZQ && __ballot(!zero16(v)) == 0) continue;
+        for (int c = 0; c < 4; ++c) v[c] = bload16(rs, off[c] + cf.fe[a]);
+        if (zq && __ballot(!zero16(v)) == 0) continue;
         z = false;
         float4 t = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
         for (int c = 0; c < 4; ++c) acc_pair(t, v[c], wa[c], wb[c]);
-        acc.x = fmaf(t.x, d2[a], acc.x);
-        acc.y = fmaf(t.y, d2[a], acc.y);
-        acc.z = fmaf(t.z, d2[a], acc.z);
-        acc.w = fmaf(t.w, d2[a], acc.w);
+        acc_face(acc, t, cf.d2[a]);
     }
     return z;
 }
@@ -361,8 +381,7 @@ __device__ __forceinline__ int level_class(float lambda, int q, float *fr) {
 
 template <int MODE>
 __device__ __forceinline__ float4 sample_class(const PyrArgs &pa, __amdgpu_buffer_rsrc_t rs, int D, float fr,
-                                               const float p[3], const uint32_t fe[3], const float d2[3],
-                                               uint32_t fmask, bool fsame) {
+                                               const float p[3], const ConeFaces &cf) {
     float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
     const int q = pa.nlevels - 1;
     if (D < 0) {
@@ -370,14 +389,18 @@ __device__ __forceinline__ float4 sample_class(const PyrArgs &pa, __amdgpu_buffe
         const int x = (int)__builtin_floorf(p[0] * (float)dim), y = (int)__builtin_floorf(p[1] * (float)dim),
                   z = (int)__builtin_floorf(p[2] * (float)dim);
         if ((unsigned)x >= (unsigned)dim || (unsigned)y >= (unsigned)dim || (unsigned)z >= (unsigned)dim) return acc;
-        const LevelInfo &L = pa.lv[0];
-        const uint4 v = bload16(rs, L.base + elem_index(L, x, y, z, 0) * 16u);
+        const SampleLevel &L = pa.lv[0];
+        uint32_t tx[2], ty[2], tz[2];
+        axis_terms((uint32_t)x + 4u, L.sx, 1u, tx);
+        axis_terms((uint32_t)y + 4u, L.sy, 4u, ty);
+        axis_terms((uint32_t)z + 4u, L.sz, 16u, tz);
+        const uint4 v = bload16(rs, L.org + (tx[0] + ty[0] + tz[0]) * 16u);
         if (MODE == 1) return make_float4(__uint_as_float(v.x), __uint_as_float(v.y), __uint_as_float(v.z),
                                           __uint_as_float(v.w));
         return unpack_h4(v.x, v.y);
     }
     if (D >= q) {
-        level_sample<MODE, false>(acc, pa.pyr, rs, pa.lv[q], p, 1.0f, fe, d2, fmask, fsame);
+        level_sample<MODE, false>(acc, pa, rs, q, p, 1.0f, cf);
         return acc;
     }
     // The coarser level first.  Its 2x2x2 cell covers the finer level's cell
@@ -386,9 +409,8 @@ __device__ __forceinline__ float4 sample_class(const PyrArgs &pa, __amdgpu_buffe
     // is zero only where every texel it filters is.  So where the coarser
     // fetch was all zero in every lane, the finer sample adds exactly 0 and is
     // skipped: cones marching through empty space.
-    const bool z = level_sample<MODE, true>(acc, pa.pyr, rs, pa.lv[D + 1], p, fr, fe, d2, fmask, fsame);
-    if (!(z && pa.nested))
-        level_sample<MODE, false>(acc, pa.pyr, rs, pa.lv[D], p, 1.0f - fr, fe, d2, fmask, fsame);
+    const bool z = level_sample<MODE, true>(acc, pa, rs, D + 1, p, fr, cf);
+    if (!(z && pa.nested)) level_sample<MODE, false>(acc, pa, rs, D, p, 1.0f - fr, cf);
     return acc;
 }
 
@@ -414,21 +436,21 @@ __device__ float4 trace_cone(const PyrArgs &pa, __amdgpu_buffer_rsrc_t rs, const
         dir[1] = dir_in[1] * il;
         dir[2] = dir_in[2] * il;
     }
-    uint32_t fe[3] = {0u, 0u, 0u};
-    float d2[3] = {0.f, 0.f, 0.f};
-    uint32_t fmask = 0u;
-    bool fsame = true;
+    ConeFaces cf = {{0u, 0u, 0u}, {0u, 0u, 0u}, {0.f, 0.f, 0.f}, 0u, true};
     if (ANISO) {
+        uint32_t fk = 0u;
 #pragma unroll
         for (int k = 0; k < 3; ++k) {
-            fe[k] = 64u * (uint32_t)(2 * k + (dir[k] >= 0.0f ? 0 : 1));
-            d2[k] = dir[k] * dir[k];
+            const uint32_t face = (uint32_t)(2 * k + (dir[k] >= 0.0f ? 0 : 1));
+            cf.fe[k] = 1024u * face;
+            cf.sfe[k] = __builtin_amdgcn_readfirstlane(cf.fe[k]);
+            cf.d2[k] = dir[k] * dir[k];
             // cones along a grid axis (faces of axis-aligned walls) weight only
             // one or two of the three faces
-            if (__ballot(d2[k] != 0.0f) != 0) fmask |= 1u << k;
+            if (__ballot(cf.d2[k] != 0.0f) != 0) cf.fmask |= 1u << k;
+            fk |= face << (4 * k);
         }
-        const uint32_t fk = fe[0] | (fe[1] << 10) | (fe[2] << 20);
-        fsame = __ballot(__builtin_amdgcn_readfirstlane(fk) != fk) == 0;
+        cf.fsame = __ballot(__builtin_amdgcn_readfirstlane(fk) != fk) == 0;
     }
     const int q = pa.nlevels - 1;
     float c0 = 0.f, c1 = 0.f, c2 = 0.f, a = 0.f;
@@ -446,9 +468,9 @@ __device__ float4 trace_cone(const PyrArgs &pa, __amdgpu_buffer_rsrc_t rs, const
             float sp[3];
 #pragma unroll
             for (int k = 0; k < 3; ++k) sp[k] = start[k] + h * ds[k];
-            if (sp[0] < 0.f || sp[0] > 1.f || sp[1] < 0.f || sp[1] > 1.f || sp[2] < 0.f || sp[2] > 1.f) break;
+            if (fminf(fminf(sp[0], sp[1]), sp[2]) < 0.f || fmaxf(fmaxf(sp[0], sp[1]), sp[2]) > 1.f) break;
             if (WARP) warp_sample_march(warp, sp);
-            const float4 smp = sample_class<MODE>(pa, rs, sched->cls[i], sched->fr[i], sp, fe, d2, fmask, fsame);
+            const float4 smp = sample_class<MODE>(pa, rs, sched->cls[i], sched->fr[i], sp, cf);
             const float aa = 1.0f - a;
             c0 += smp.x * aa;
             c1 += smp.y * aa;
@@ -464,7 +486,7 @@ __device__ float4 trace_cone(const PyrArgs &pa, __amdgpu_buffer_rsrc_t rs, const
         float sp[3];
 #pragma unroll
         for (int k = 0; k < 3; ++k) sp[k] = start[k] + (h * dir[k]) * scale;
-        if (sp[0] < 0.f || sp[0] > 1.f || sp[1] < 0.f || sp[1] > 1.f || sp[2] < 0.f || sp[2] > 1.f) break;
+        if (fminf(fminf(sp[0], sp[1]), sp[2]) < 0.f || fmaxf(fmaxf(sp[0], sp[1]), sp[2]) > 1.f) break;
         if (WARP) warp_sample_march(warp, sp);
         float fr;
         const int D = level_class(lod + lod_offset, q, &fr);
@@ -472,7 +494,7 @@ __device__ float4 trace_cone(const PyrArgs &pa, __amdgpu_buffer_rsrc_t rs, const
         if (ULOD) {
             const int Du = __builtin_amdgcn_readfirstlane(D);
             const float fru = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(fr)));
-            smp = sample_class<MODE>(pa, rs, Du, fru, sp, fe, d2, fmask, fsame);
+            smp = sample_class<MODE>(pa, rs, Du, fru, sp, cf);
         } else {
             smp = make_float4(0.f, 0.f, 0.f, 0.f);
             bool pending = true;
@@ -481,7 +503,7 @@ __device__ float4 trace_cone(const PyrArgs &pa, __amdgpu_buffer_rsrc_t rs, const
                 if (m == 0) break;
                 const int Du = __builtin_amdgcn_readlane(D, __builtin_ctzll(m));
                 if (pending && D == Du) {
-                    smp = sample_class<MODE>(pa, rs, Du, fr, sp, fe, d2, fmask, fsame);
+                    smp = sample_class<MODE>(pa, rs, Du, fr, sp, cf);
                     pending = false;
                 }
             }
@@ -504,76 +526,95 @@ static __constant__ float kConeDirs[6][3] = {{0.0f, 1.0f, 0.0f},
                                       {-0.823639f, 0.5f, 0.267617f}};
 static __constant__ float kConeW[6] = {0.25f, 0.15f, 0.15f, 0.15f, 0.15f, 0.15f};
 
-// One pixel of the phong.frag gather: 6 diffuse cones (+ the specular cone).
-template <int MODE, bool ANISO, bool WARP>
-__device__ __forceinline__ void trace_pixel(const TraceLaunch &t, const PyrArgs &pa, __amdgpu_buffer_rsrc_t rs, int px,
-                                            int py, bool reflections) {
-    const size_t pi = (size_t)py * t.width + px;
+// A G-buffer texel as the gather uses it: texture-space position, unit normal,
+// tangent frame.
+struct TracePixel {
+    float gp[3], pos[3], N[3], nraw[3], T[3], B[3], rough;
+    bool covered;
+};
+__device__ __forceinline__ void load_pixel(const TraceLaunch &t, size_t pi, TracePixel &x) {
     const float4 *g = (const float4 *)&t.gbuf[pi];
     const float4 g0 = g[0], g1 = g[1], g2 = g[2], g3 = g[3];
-    if (__float_as_uint(g2.w) == 0u) {
-        t.out_ind[pi] = make_float4(0.f, 0.f, 0.f, 0.f);
-        if (reflections) t.out_spec[pi] = make_float4(0.f, 0.f, 0.f, 0.f);
-        return;
-    }
-    float pos[3];
-    const float gp[3] = {g0.x, g0.y, g0.z};
+    x.covered = __float_as_uint(g2.w) != 0u;
+    x.gp[0] = g0.x;
+    x.gp[1] = g0.y;
+    x.gp[2] = g0.z;
 #pragma unroll
-    for (int k = 0; k < 3; ++k) pos[k] = ((gp[k] - t.ext.center[k]) - t.ext.vmin[k]) / (t.ext.vmax[k] - t.ext.vmin[k]);
-    const float nraw[3] = {g1.x, g1.y, g1.z};
-    const float T[3] = {g2.x, g2.y, g2.z};
-    const float B[3] = {g3.x, g3.y, g3.z};
-    float N[3];
-    nrm3(nraw, N);
-    float i0 = 0.f, i1 = 0.f, i2 = 0.f, i3 = 0.f;
-    for (int i = 0; i < 6; ++i) {
-        const float cx = kConeDirs[i][0], cy = kConeDirs[i][1], cz = kConeDirs[i][2];
-        float d[3];
+    for (int k = 0; k < 3; ++k) x.pos[k] = ((x.gp[k] - t.ext.center[k]) - t.ext.vmin[k]) / (t.ext.vmax[k] - t.ext.vmin[k]);
+    x.nraw[0] = g1.x;
+    x.nraw[1] = g1.y;
+    x.nraw[2] = g1.z;
+    x.rough = g1.w;
+    x.T[0] = g2.x;
+    x.T[1] = g2.y;
+    x.T[2] = g2.z;
+    x.B[0] = g3.x;
+    x.B[1] = g3.y;
+    x.B[2] = g3.z;
+    nrm3(x.nraw, x.N);
+}
+
+// Diffuse cone i of the gather (phong.frag:480-484).
+template <int MODE, bool ANISO, bool WARP>
+__device__ __forceinline__ float4 diffuse_cone(const TraceLaunch &t, const PyrArgs &pa, __amdgpu_buffer_rsrc_t rs,
+                                               const TracePixel &x, int i) {
+    const float cx = kConeDirs[i][0], cy = kConeDirs[i][1], cz = kConeDirs[i][2];
+    float d[3];
 #pragma unroll
-        for (int k = 0; k < 3; ++k) d[k] = (T[k] * cx + B[k] * cy) + nraw[k] * cz;
-        const float4 r = trace_cone<MODE, ANISO, true, WARP>(pa, rs, pos, N, d, t.d_steps, t.d_bias, t.d_tan_half, t.d_h0,
-                                                       t.d_lod_offset, t.warp, &t.d_sched);
-        const float w = kConeW[i];
-        i0 += w * r.x;
-        i1 += w * r.y;
-        i2 += w * r.z;
-        i3 += w * r.w;
-    }
-    const float occ = 1.0f - clampf(i3, 0.0f, 1.0f);
+    for (int k = 0; k < 3; ++k) d[k] = (x.T[k] * cx + x.B[k] * cy) + x.nraw[k] * cz;
+    return trace_cone<MODE, ANISO, true, WARP>(pa, rs, x.pos, x.N, d, t.d_steps, t.d_bias, t.d_tan_half, t.d_h0,
+                                               t.d_lod_offset, t.warp, &t.d_sched);
+}
+
+// The weighted sum of the diffuse cones, one cone at a time in order, and its
+// image value (phong.frag:483-489).
+__device__ __forceinline__ void add_cone(float4 &sum, const float4 &r, int i) {
+    const float w = kConeW[i];
+    sum.x += w * r.x;
+    sum.y += w * r.y;
+    sum.z += w * r.z;
+    sum.w += w * r.w;
+}
+__device__ __forceinline__ float4 indirect_value(const TraceLaunch &t, const float4 &sum) {
+    const float occ = 1.0f - clampf(sum.w, 0.0f, 1.0f);
     const float m = t.draw_occlusion ? occ : 1.0f;
-    t.out_ind[pi] = make_float4(i0 * m, i1 * m, i2 * m, occ);
-    if (reflections) {
-        float angle = t.s_angle;
-        if (t.angle_from_roughness && t.has_roughness) angle = (g1.w * 3.1415982f) * 0.1f;  // PI of common.glsl:1
-        const float I[3] = {gp[0] - t.eye[0], gp[1] - t.eye[1], gp[2] - t.eye[2]};
-        const float dni = dot3(N, I);
-        float R[3];
+    return make_float4(sum.x * m, sum.y * m, sum.z * m, occ);
+}
+
+// The specular cone (phong.frag:491-512).
+template <int MODE, bool ANISO, bool WARP>
+__device__ __forceinline__ float4 specular_cone(const TraceLaunch &t, const PyrArgs &pa, __amdgpu_buffer_rsrc_t rs,
+                                                const TracePixel &x) {
+    float angle = t.s_angle;
+    if (t.angle_from_roughness && t.has_roughness) angle = (x.rough * 3.1415982f) * 0.1f;  // PI of common.glsl:1
+    const float I[3] = {x.gp[0] - t.eye[0], x.gp[1] - t.eye[1], x.gp[2] - t.eye[2]};
+    const float dni = dot3(x.N, I);
+    float R[3];
 #pragma unroll
-        for (int k = 0; k < 3; ++k) R[k] = I[k] - (2.0f * dni) * N[k];
-        const float th = tanf(angle / 2.0f);
-        // One material under the whole wavefront (the usual case): every lane's
-        // cone has the same aperture, so the step schedule and the level
-        // classes are the same in every lane.
-        const float th0 = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(th)));
-        float4 r;
-        if (__ballot(__float_as_int(th) != __float_as_int(th0)) == 0)
-            r = trace_cone<MODE, ANISO, true, WARP>(pa, rs, pos, N, R, t.s_steps, t.s_bias, th, t.s_h0, t.s_lod_offset,
-                                              t.warp);
-        else
-            r = trace_cone<MODE, ANISO, false, WARP>(pa, rs, pos, N, R, t.s_steps, t.s_bias, th, t.s_h0, t.s_lod_offset,
-                                               t.warp);
-        t.out_spec[pi] = r;
-    }
+    for (int k = 0; k < 3; ++k) R[k] = I[k] - (2.0f * dni) * x.N[k];
+    const float th = tanf(angle / 2.0f);
+    // One material under the whole wavefront (the usual case): every lane's
+    // cone has the same aperture, so the step schedule and the level classes
+    // are the same in every lane.
+    const float th0 = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(th)));
+    if (__ballot(__float_as_int(th) != __float_as_int(th0)) == 0)
+        return trace_cone<MODE, ANISO, true, WARP>(pa, rs, x.pos, x.N, R, t.s_steps, t.s_bias, th, t.s_h0,
+                                                   t.s_lod_offset, t.warp);
+    return trace_cone<MODE, ANISO, false, WARP>(pa, rs, x.pos, x.N, R, t.s_steps, t.s_bias, th, t.s_h0, t.s_lod_offset,
+                                                t.warp);
 }
 
 inline PyrArgs pyr_args(const PyrDesc &pyr, int nested) {
     PyrArgs a;
     a.pyr = pyr.pyr;
     a.bytes = pyr.bytes;
-    a.lv = pyr.d_lv;
     a.dim = pyr.dim;
     a.nlevels = pyr.nlevels;
     a.nested = nested;
+    for (int l = 0; l < VCT_MAX_LEVELS; ++l) {
+        const LevelInfo &L = pyr.lv[l < pyr.nlevels ? l : 0];
+        a.lv[l] = SampleLevel{(float)L.size, L.stage - L.pad * 16u, L.sx, L.sy, L.sz, L.nfaces, L.fmt != 0 ? 1 : 0, 0};
+    }
     return a;
 }
 

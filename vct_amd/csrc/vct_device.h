@@ -224,55 +224,6 @@ __device__ __forceinline__ float4 load_texel(const char *pyr, const float *scale
     return unpack_h4(v.x, v.y);
 }
 
-// GL LINEAR inside face 0 of one level (border 0), FP32 weights and sums.
-// p in [0,1]^3 texture coordinates; s = the level's edge.
-__device__ __forceinline__ float4 level_linear(const char *pyr, const LevelInfo &L, const float p[3]) {
-    const int s = L.size;
-    int i0[3];
-    float f[3];
-    for (int k = 0; k < 3; ++k) {
-        const float u = p[k] * (float)s - 0.5f;
-        const float fl = __builtin_floorf(u);
-        i0[k] = (int)fl;
-        f[k] = u - fl;
-    }
-    float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (L.fmt == 0) {  // fp16 pairs: one load per (y, z) corner pair
-        const bool xin = i0[0] >= 0 && i0[0] < s;  // i0 = s - 1 reads the zero border half
-        const bool xneg = i0[0] == -1;
-        if (!xin && !xneg) return acc;
-        const int cx = xneg ? 0 : i0[0];
-        const float wlo = xneg ? f[0] : 1.0f - f[0], whi = xneg ? 0.0f : f[0];
-        for (int c = 0; c < 4; ++c) {
-            const int dy = c & 1, dz = c >> 1;
-            const int y = i0[1] + dy, z = i0[2] + dz;
-            if ((unsigned)y >= (unsigned)s || (unsigned)z >= (unsigned)s) continue;
-            const float wyz = (dy ? f[1] : 1.0f - f[1]) * (dz ? f[2] : 1.0f - f[2]);
-            const uint4 v = *(const uint4 *)(pyr + L.base + (size_t)elem_index(L, cx, y, z, 0) * 16);
-            const float4 lo = unpack_h4(v.x, v.y), hi = unpack_h4(v.z, v.w);
-            const float a = wlo * wyz, b = whi * wyz;
-            acc.x += a * lo.x + b * hi.x;
-            acc.y += a * lo.y + b * hi.y;
-            acc.z += a * lo.z + b * hi.z;
-            acc.w += a * lo.w + b * hi.w;
-        }
-        return acc;
-    }
-    for (int c = 0; c < 8; ++c) {
-        const int dx = c & 1, dy = (c >> 1) & 1, dz = c >> 2;
-        const int x = i0[0] + dx, y = i0[1] + dy, z = i0[2] + dz;
-        if ((unsigned)x >= (unsigned)s || (unsigned)y >= (unsigned)s || (unsigned)z >= (unsigned)s) continue;
-        const float w = ((dx ? f[0] : 1.0f - f[0]) * (dy ? f[1] : 1.0f - f[1])) * (dz ? f[2] : 1.0f - f[2]);
-        // fp32 elements, or the decoded copy of an fp8 level
-        const float4 t = *(const float4 *)(pyr + L.stage + (size_t)elem_index(L, x, y, z, 0) * 16);
-        acc.x += w * t.x;
-        acc.y += w * t.y;
-        acc.z += w * t.z;
-        acc.w += w * t.w;
-    }
-    return acc;
-}
-
 // GL LINEAR sample of an fp32 depth texture, CLAMP_TO_BORDER with border 1.0
 // (src/Application.cpp:46-53), with a textureOffset texel offset.
 __device__ __forceinline__ float shadow_bilinear(const float *__restrict__ sm, int N, float s, float t, int ox,
