@@ -119,45 +119,54 @@ __global__ __launch_bounds__(256) void k_block_slots(const uint64_t *__restrict_
     }
 }
 
-// The large triangles of a walk: one wavefront per 8x8-pixel block of a
-// triangle's bounding box, its lanes the block's pixels (row-major).  Each
-// wavefront takes a contiguous run of blocks, so consecutive blocks mostly
-// belong to one triangle and its record (wave-uniform) is read again only when
-// the run enters the next triangle (its slot from k_block_slots, or the same
-// search past that table).  Each lane's edge values are the block corner's
-// (wave-uniform) plus the lane's offset A_i dx + B_i dy, set once per triangle:
-// in 32-bit wrapping arithmetic for the small form (the same value modulo 2^32
-// as edge_value's sum), in FP64 for the 64-bit form (every term is an integer
-// below 2^53, so each sum is exact).  The barycentrics are quot_f32(E, area)
-// with the triangle's reciprocal, so every fragment and its barycentrics are
-// those the pixel walk produces.  F provides enter(slot, edges) (the slot's
-// wave-uniform data, and the image size W x H) and frag(edges, px, py, l).
+// The large triangles of a walk, 8x8-pixel blocks of their bounding boxes, the
+// lanes a block's pixels (row-major).  A wavefront takes runs of consecutive
+// blocks (up to kBlockRun; run r by wavefront r % wavefronts, so that the runs
+// of covered blocks and of empty ones are dealt out evenly), and a triangle's
+// record is wave-uniform (its slot from k_block_slots, or the same search past
+// that table).  Each lane keeps its three edge values in FP64 and steps them
+// from block to block: every one is an integer below 2^53 (|A|, |B| <= 2^28, a
+// coordinate in 1/256 px below 2^22), so every sum is exact, the values are
+// those of edge_value in both of its forms, and the barycentrics are
+// quot_f32(E, area) with the triangle's reciprocal: every fragment and its
+// barycentrics are those the pixel walk produces.  F provides Tri (a triangle's
+// wave-uniform data, the image size W x H among it), enter(slot, edges) that
+// gives it, and three stages of a fragment, between which a Pending goes:
+// fetch(tri, px, py, in), depth(tri, l, pending) and store(pending), which runs
+// after the wavefront's next covered block has been fetched.
+//
+// What bounds it: VALU issue and the scalar work beside it (an empty block 3
+// additions and 3 comparisons, a covered one 12 more for the quotients and 8
+// for the depth), then the atomics, which a load of the word before them spares
+// where a nearer fragment is already there.  It was 20 and 45 vector
+// instructions a block, in two forms (32-bit and FP64) whose arrays took 82
+// registers: 5 wavefronts per SIMD for a grid of 8, on equal shares of
+// consecutive blocks.  Five 1024^2 maps: 286 us before, 183; five 2048^2 maps:
+// 1024 us before, 534.  The load in the same stage as the atomic suits the depth
+// maps (190 and 560 us with the G-buffer's stages); the G-buffer, fewer blocks
+// of longer triangles, waits for the load, so the atomic goes one block later
+// (1920x1080: 79 us without the load, 92 with it, 73 one block later; 3840x2160:
+// 427, 271, 254).
+
+constexpr int kBlockRun = 64;
+
 template <class F>
-__global__ __launch_bounds__(256) void k_raster_blocks(const int4 *__restrict__ recs, const uint64_t *__restrict__ offs,
-                                                       const uint32_t *__restrict__ chunk, size_t chunk_cap, int nslots,
-                                                       const uint32_t *__restrict__ bslots, size_t bslots_cap, F fr) {
-    F f = fr;
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void k_raster_blocks(
+    const int4 *__restrict__ recs, const uint64_t *__restrict__ offs, const uint32_t *__restrict__ chunk,
+    size_t chunk_cap, int nslots, const uint32_t *__restrict__ bslots, size_t bslots_cap, F f) {
     const uint64_t total = offs[nslots];
     const uint64_t nchunks = (total + 63) >> 6;
     const int lane = threadIdx.x & 63;
-    const uint64_t nwaves = ((uint64_t)gridDim.x * blockDim.x) >> 6;
-    const uint64_t wave = __builtin_amdgcn_readfirstlane((uint32_t)(((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6));
-    const uint64_t per = (total + nwaves - 1) / nwaves;
-    const uint64_t k0 = wave * per, k1 = k0 + per < total ? k0 + per : total;
-    uint64_t run_lo = 0, run_hi = 0;  // the blocks [run_lo, run_hi) of the current slot
-    int slot = 0;
-    Edges e;
-    uint32_t nbx = 1, bxi = 0, byi = 0;  // the block's column and row in the triangle's bounding box
-    double rcp = 0.0;                    // RN64(1 / area)
-    uint32_t off32[3] = {0u, 0u, 0u};    // small form: A_i dx + B_i dy of this lane (mod 2^32)
-    double offd[3] = {0.0, 0.0, 0.0}, Ad[3] = {0.0, 0.0, 0.0}, Bd[3] = {0.0, 0.0, 0.0}, Cd[3] = {0.0, 0.0, 0.0};
-    const int dxl = (lane & 7) * 256, dyl = (lane >> 3) * 256;
-    for (uint64_t k = k0; k < k1; ++k, ++bxi) {
-        if (bxi == nbx) {
-            bxi = 0;
-            ++byi;
-        }
-        if (k >= run_hi) {  // the run enters the next triangle
+    const uint32_t nwaves = (gridDim.x * blockDim.x) >> 6;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
+    const uint64_t share = (total + nwaves - 1) / nwaves;
+    const uint64_t run = share < (uint64_t)kBlockRun ? (share ? share : 1) : (uint64_t)kBlockRun;
+    typename F::Pending last = {};
+    const double dxl = (double)((lane & 7) * 256 + 128), dyl = (double)((lane >> 3) * 256 + 128);
+    for (uint64_t r0 = wave * run; r0 < total; r0 += nwaves * run) {
+        const uint64_t r1 = r0 + run < total ? r0 + run : total;
+        uint64_t k = r0;
+        while (k < r1) {  // the run's next triangle
             int lo;
             if (k < bslots_cap) {
                 lo = (int)bslots[k];
@@ -171,81 +180,102 @@ __global__ __launch_bounds__(256) void k_raster_blocks(const int4 *__restrict__ 
                     else hi = mid - 1;
                 }
             }
-            slot = __builtin_amdgcn_readfirstlane(lo);
-            run_lo = offs[slot];
-            run_hi = offs[slot + 1];
+            const int slot = __builtin_amdgcn_readfirstlane(lo);
+            const uint64_t t0 = offs[slot], t1 = offs[slot + 1];
+            const uint32_t n = (uint32_t)((t1 < r1 ? t1 : r1) - k);  // its blocks in this run
+            Edges e;
             load_edges(recs, (size_t)slot, e);
-            f.enter(slot, e);
-            nbx = (uint32_t)(((e.x0 + e.bw - 1) >> 3) - (e.x0 >> 3) + 1);
-            const uint32_t local = (uint32_t)(k - run_lo);  // the run may enter a triangle mid-way
-            bxi = local % nbx;
-            byi = local / nbx;
-            rcp = 1.0 / (double)e.area;
+            const typename F::Tri tri = f.enter(slot, e);
+            const uint32_t nbx = (uint32_t)(((e.x0 + e.bw - 1) >> 3) - (e.x0 >> 3) + 1);
+            const uint32_t local = (uint32_t)(k - t0);  // the run may enter a triangle mid-way
+            uint32_t bxi = __builtin_amdgcn_readfirstlane(local % nbx);
+            const int bx0 = (e.x0 >> 3) * 8, by = ((e.y0 >> 3) + (int)(local / nbx)) * 8;
+            const double rcp = 1.0 / (double)e.area;  // RN64(1 / area)
+            double E[3], row[3], As[3], Bs[3], lim[3];
 #pragma unroll
             for (int i = 0; i < 3; ++i) {
-                if (e.small) {
-                    off32[i] = (uint32_t)e.A[i] * (uint32_t)dxl + (uint32_t)e.B[i] * (uint32_t)dyl;
+                const double A = (double)e.A[i], B = (double)e.B[i];
+                // the small form's edge value at the bounding box corner, as the
+                // value at the origin
+                const double C = e.small ? (double)e.E0[i] - (A * (double)(e.x0 << 8) + B * (double)(e.y0 << 8))
+                                         : (double)e.C[i];
+                row[i] = fma(A, (double)(bx0 * 256) + dxl, fma(B, (double)(by * 256) + dyl, C));
+                As[i] = A * 2048.0;
+                Bs[i] = B * 2048.0;
+                E[i] = fma((double)(int)bxi, As[i], row[i]);
+                lim[i] = (double)(-e.bias[i]);
+            }
+            int px = bx0 + (int)bxi * 8 + (lane & 7), py = by + (lane >> 3);
+            for (uint32_t j = 0; j < n; ++j) {
+                // px, py: outside where the block overhangs the image
+                const bool in = (E[0] >= lim[0]) & (E[1] >= lim[1]) & (E[2] >= lim[2]) & (px < tri.W) & (py < tri.H);
+                if (__ballot(in) != 0) {  // an empty block ends here
+                    typename F::Pending cur = f.fetch(tri, px, py, in);
+                    float l[3];
+#pragma unroll
+                    for (int i = 0; i < 3; ++i) l[i] = quot_f32((float)E[i], rcp);
+                    f.depth(tri, l, cur);
+                    f.store(last);  // the last covered block's: its word has arrived by now
+                    last = cur;
+                }
+                if (++bxi == nbx) {
+                    bxi = 0;
+                    px = bx0 + (lane & 7);
+                    py += 8;
+#pragma unroll
+                    for (int i = 0; i < 3; ++i) E[i] = row[i] = row[i] + Bs[i];
                 } else {
-                    Ad[i] = (double)e.A[i];
-                    Bd[i] = (double)e.B[i];
-                    Cd[i] = (double)e.C[i];
-                    offd[i] = Ad[i] * (double)dxl + Bd[i] * (double)dyl;
+                    px += 8;
+#pragma unroll
+                    for (int i = 0; i < 3; ++i) E[i] = E[i] + As[i];
                 }
             }
+            k += n;
         }
-        const int bx = ((e.x0 >> 3) + (int)bxi) * 8, by = ((e.y0 >> 3) + (int)byi) * 8;
-        const int px = bx + (lane & 7), py = by + (lane >> 3);
-        if (px >= f.W || py >= f.H) continue;  // the block overhangs the image
-        float l[3];
-        bool in = true;
-        if (e.small) {
-            // edge_value's dx = ((px - x0) << 8) + 128 = cx + dxl, likewise dy
-            const uint32_t cx = (uint32_t)(((bx - e.x0) << 8) + 128), cy = (uint32_t)(((by - e.y0) << 8) + 128);
-            int32_t E[3];
-#pragma unroll
-            for (int i = 0; i < 3; ++i) {
-                const uint32_t corner = (uint32_t)e.E0[i] + (uint32_t)e.A[i] * cx + (uint32_t)e.B[i] * cy;
-                E[i] = (int32_t)(corner + off32[i]);
-                in = in && ((int32_t)((uint32_t)E[i] + (uint32_t)e.bias[i]) >= 0);
-            }
-            if (!in) continue;
-#pragma unroll
-            for (int i = 0; i < 3; ++i) l[i] = quot_f32((float)E[i], rcp);
-        } else {
-            const double sx = (double)(bx * 256 + 128), sy = (double)(by * 256 + 128);
-            double E[3];
-#pragma unroll
-            for (int i = 0; i < 3; ++i) {
-                E[i] = fma(Ad[i], sx, fma(Bd[i], sy, Cd[i])) + offd[i];
-                in = in && (E[i] >= (double)(-e.bias[i]));
-            }
-            if (!in) continue;
-#pragma unroll
-            for (int i = 0; i < 3; ++i) l[i] = quot_f32((float)E[i], rcp);
-        }
-        f.frag(e, px, py, l);
     }
+    f.store(last);
 }
 
-// ShadowFrag for the block walk.
+// A walk's shadow maps by light index (Edges::user), in the kernel arguments.
+struct ShadowMaps {
+    uint32_t *map[kMaxLights];
+    int size[kMaxLights];
+};
+typedef __attribute__((address_space(1))) uint32_t global_u32;
+
+// ShadowFrag for the block walk: load, comparison and atomic in one stage.
 struct ShadowBlockFrag {
     const float4 *attr;
-    const DevLight *lights;
-    float4 a;
-    uint32_t *map;
-    int W, H;
-    __device__ void enter(int slot, const Edges &e) {
-        a = attr[slot];
-        const DevLight &L = lights[e.user];
-        map = (uint32_t *)const_cast<float *>(L.shadowmap);
-        W = H = (int)L.shadow_size;
+    ShadowMaps maps;
+    struct Tri {
+        float4 a;
+        global_u32 *map;
+        int W, H;
+    };
+    struct Pending {
+        global_u32 *d;
+        bool live;
+    };
+    __device__ Tri enter(int slot, const Edges &e) const {
+        Tri t;
+        t.a = attr[slot];
+        t.map = (global_u32 *)maps.map[e.user];
+        t.W = t.H = maps.size[e.user];
+        return t;
     }
-    __device__ void frag(const Edges &, int px, int py, const float l[3]) {
-        float z = interp3(l, a.x, a.y, a.z);
+    __device__ Pending fetch(const Tri &t, int px, int py, bool in) const {
+        return Pending{t.map + (uint32_t)(py * t.W + px), in};
+    }
+    __device__ void depth(const Tri &t, const float l[3], Pending &p) const {
+        float z = interp3(l, t.a.x, t.a.y, t.a.z);
         z = z + 0.0f;
-        if (!(z >= 0.0f && z <= 1.0f)) return;
-        atomicMin(&map[(size_t)py * W + px], __float_as_uint(z));
+        if (p.live && z >= 0.0f && z <= 1.0f) {
+            const uint32_t zu = __float_as_uint(z);
+            if (__hip_atomic_load(p.d, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) > zu)  // seen()
+                __hip_atomic_fetch_min(p.d, zu, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
     }
+    __device__ void store(const Pending &) const {}
 };
 
 struct ShadowFrag {
@@ -296,7 +326,13 @@ hipError_t launch_shadowmaps(const DevScene &sc, const DevLight *hlights, const 
             hipLaunchKernelGGL(k_block_slots, dim3(kRasterBlocks), dim3(256), 0, s, rs.boffs, rs.bchunk, rs.chunk_cap,
                                (int)nslots, rs.bslots, rs.bslots_cap);
             if ((e = hipGetLastError()) != hipSuccess) return e;
-            ShadowBlockFrag fb{rs.attr, dlights, make_float4(0.f, 0.f, 0.f, 0.f), nullptr, 0, 0};
+            ShadowBlockFrag fb{};
+            fb.attr = rs.attr;
+            for (int j = 0; j < nb; ++j) {
+                const DevLight &L = hlights[li[j0 + j]];
+                fb.maps.map[li[j0 + j]] = (uint32_t *)const_cast<float *>(L.shadowmap);
+                fb.maps.size[li[j0 + j]] = (int)L.shadow_size;
+            }
             hipLaunchKernelGGL(k_raster_blocks<ShadowBlockFrag>, dim3(kRasterBlocks), dim3(256), 0, s, rs.rec,
                                rs.boffs, rs.bchunk, rs.chunk_cap, (int)nslots, rs.bslots, rs.bslots_cap, fb);
             if ((e = hipGetLastError()) != hipSuccess) return e;
@@ -444,16 +480,32 @@ struct GbufBlockFrag {
     const float4 *attr;
     unsigned long long *vis;
     int W, H;
-    float4 a;
-    __device__ void enter(int slot, const Edges &) { a = attr[slot]; }
-    __device__ void frag(const Edges &e, int px, int py, const float l[3]) {
-        float z = interp3(l, a.x, a.y, a.z);
+    struct Tri {
+        float4 a;
+        uint32_t low;  // the key's low word: ~triangle
+        int W, H;
+    };
+    struct Pending {
+        unsigned long long *d, key, seen;
+        bool live;
+    };
+    __device__ Tri enter(int slot, const Edges &e) const { return Tri{attr[slot], 0xffffffffu - (uint32_t)e.user, W, H}; }
+    __device__ Pending fetch(const Tri &, int px, int py, bool in) const {
+        Pending p;
+        p.d = &vis[(size_t)(uint32_t)(py * W + px)];
+        p.key = p.seen = 0ull;
+        p.live = in;
+        if (in) p.seen = vctk::seen(p.d);
+        return p;
+    }
+    __device__ void depth(const Tri &t, const float l[3], Pending &p) const {
+        float z = interp3(l, t.a.x, t.a.y, t.a.z);
         z = z + 0.0f;
-        if (!(z >= 0.0f && z <= 1.0f)) return;
-        const uint32_t tri = (uint32_t)e.user;
-        const unsigned long long key =
-            ((unsigned long long)__float_as_uint(z) << 32) | (unsigned long long)(0xffffffffu - tri);
-        atomicMin(&vis[(size_t)py * W + px], key);
+        p.live = p.live && z >= 0.0f && z <= 1.0f;
+        p.key = ((unsigned long long)__float_as_uint(z) << 32) | (unsigned long long)t.low;
+    }
+    __device__ void store(const Pending &p) const {
+        if (p.live && p.seen > p.key) atomicMin(p.d, p.key);
     }
 };
 
@@ -582,7 +634,7 @@ hipError_t launch_gbuffer(const DevScene &sc, const vct_camera &cam, uint64_t *v
         hipLaunchKernelGGL(k_block_slots, dim3(kRasterBlocks), dim3(256), 0, s, rs.boffs, rs.bchunk, rs.chunk_cap,
                            (int)nslots, rs.bslots, rs.bslots_cap);
         if ((e = hipGetLastError()) != hipSuccess) return e;
-        GbufBlockFrag fb{rs.attr, (unsigned long long *)vis, cam.width, cam.height, make_float4(0.f, 0.f, 0.f, 0.f)};
+        GbufBlockFrag fb{rs.attr, (unsigned long long *)vis, cam.width, cam.height};
         hipLaunchKernelGGL(k_raster_blocks<GbufBlockFrag>, dim3(kRasterBlocks), dim3(256), 0, s, rs.rec, rs.boffs,
                            rs.bchunk, rs.chunk_cap, (int)nslots, rs.bslots, rs.bslots_cap, fb);
         if ((e = hipGetLastError()) != hipSuccess) return e;

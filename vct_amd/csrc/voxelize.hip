@@ -682,8 +682,11 @@ __global__ __launch_bounds__(256) void k_tess_points(DevScene sc, TessArgs ta, c
         }
         const uint32_t vi = grid_index(idx[0], idx[1], idx[2], ta.dim >> 2);
         if (accum == VCT_ACCUM_MAX) {
-            atomicMax(&albedo[vi], pack_unorm4x8(col.x, col.y, col.z, col.w));
-            atomicMax(&normal[vi], pack_unorm4x8(ne0, ne1, ne2, 1.0f));
+            // many points fall into a voxel that already holds more: 181 us for the
+            // icospheres without the loads, 133 with them (256^3)
+            const uint32_t pa = pack_unorm4x8(col.x, col.y, col.z, col.w), pn = pack_unorm4x8(ne0, ne1, ne2, 1.0f);
+            if (seen(&albedo[vi]) < pa) atomicMax(&albedo[vi], pa);
+            if (seen(&normal[vi]) < pn) atomicMax(&normal[vi], pn);
         } else {
             rgba8_avg(&albedo[vi], col.x, col.y, col.z);
             rgba8_avg(&normal[vi], ne0, ne1, ne2);
