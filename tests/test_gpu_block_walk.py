@@ -60,3 +60,34 @@ def test_block_walk_edges(n):
             assert np.array_equal(got.view(np.uint32), ob.gbuffer(sc, cam).view(np.uint32)), (n, w, h)
     finally:
         app.close()
+
+
+@pytest.mark.parametrize("n", [2047, 2048, 2049, 16384, 16385])
+def test_slot_counts(n):
+    """Item offsets at the edges of a tile of slots and of the count up to
+    which a tile adds up the slots in front of it itself, small triangles and
+    a few that cover the whole map (more chunks of items than slots)."""
+    app = make_app(1, dim=32)
+    try:
+        ctx, fs = app.ctx, app.frame_state(0)
+        eye = np.eye(4, dtype=np.float32)[None]
+        m = _soup(app.mesh()["pos"], n, n)
+        c = m["pos"].mean(1, keepdims=True)
+        keep = np.random.default_rng(1).random((n, 1, 1)) < 0.995
+        m["pos"] = np.where(keep, c + (m["pos"] - c) * np.float32(0.02), m["pos"]).astype(np.float32)
+        ctx.set_scene(m["pos"], m["nrm"], m["tan"], m["albedo"], m["obj"], 1)
+        ctx.set_transforms(eye)
+        sc = ob.SceneArrays(m, eye)
+        L = abi.Light.from_buffer_copy(next(L for L in fs["lights"] if L.shadow_caster))
+        L.shadow_size = 200
+        ctx.set_lights([L])
+        ctx.shadowmaps()
+        ref = ob.shadowmap(sc, L)
+        assert (ref < 1.0).any()
+        assert np.array_equal(ctx.shadow(0).view(np.uint32), ref.view(np.uint32))
+        ctx.voxelize(fs["vox"])
+        alb, nrm, st = ob.voxelize(sc, [L], [ref], fs["vox"], 32)
+        assert np.array_equal(ctx.albedo(), alb) and np.array_equal(ctx.normal(), nrm)
+        assert ctx.stats().total_voxel_fragments == st.total_voxel_fragments
+    finally:
+        app.close()

@@ -438,7 +438,6 @@ void vct_destroy(vct_ctx *c) {
     dfree(c->rs.bcounts);
     dfree(c->rs.boffs);
     dfree(c->rs.bchunk);
-    dfree(c->rs.bslots);
     dfree(c->rs.tsum);
     dfree(c->d_gbuf);
     dfree(c->d_vis);
@@ -541,8 +540,6 @@ static int ensure_raster(vct_ctx *c, size_t slots) {
         c->rs.chunk_cap = (size_t)1 << 22;  // chunk starts for 256M items; beyond that a full search is used
         HIPCHK(c, dalloc(&c->rs.chunk, c->rs.chunk_cap * sizeof(uint32_t)));
         HIPCHK(c, dalloc(&c->rs.bchunk, c->rs.chunk_cap * sizeof(uint32_t)));
-        c->rs.bslots_cap = (size_t)1 << 24;  // 64 MiB: blocks past this use the walk's own search
-        HIPCHK(c, dalloc(&c->rs.bslots, c->rs.bslots_cap * sizeof(uint32_t)));
     }
     c->rs.cap_slots = slots;
     return VCT_OK;

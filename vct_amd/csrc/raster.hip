@@ -11,6 +11,8 @@
 // after the pre-pass does.
 #pragma clang fp contract(off)
 
+#include <algorithm>
+
 #include "raster_common.h"
 #include "texture.h"
 
@@ -50,13 +52,31 @@ __device__ __forceinline__ uint64_t bbox_blocks(const int4 r[4], uint64_t cnt) {
     return nbx * nby;
 }
 
+// Words of `w` to v, by `threads` threads of which this is the t-th: 16 bytes
+// at a time (w is the start of an allocation).
+__device__ __forceinline__ void fill_words(uint32_t *w, uint32_t v, size_t n, size_t t, size_t threads) {
+    for (size_t i = t; i < n / 4; i += threads) ((uint4 *)w)[i] = make_uint4(v, v, v, v);
+    if (t < (n & 3)) w[(n & ~(size_t)3) + t] = v;
+}
+
+// Workgroups of a set-up kernel that also clears `words` words of an image: its
+// triangles', and no fewer than the clear fills (4 stores a thread, up to 4
+// workgroups per CU).  The clear's writes run beside the set-up's own work: five
+// 1024^2 maps took 5 launches of 5.7 us before, now 4 us of the set-up's.
+inline unsigned setup_blocks(int ntri, size_t words) {
+    const size_t tri = ((size_t)ntri + 255) / 256, fill = (words + 4095) / 4096;
+    return (unsigned)std::max(tri, std::min(fill, (size_t)1024));
+}
+
 __global__ __launch_bounds__(256) void k_shadow_setup(DevScene sc, const DevLight *__restrict__ lights, uint64_t li,
                                                       int4 *rec, float4 *attr, uint32_t *counts, uint32_t *bcounts) {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= sc.ntri) return;
     const int l = (int)((li >> (5u * blockIdx.y)) & 31u);
     const float *ls = lights[l].ls;
     const int N = (int)lights[l].shadow_size;
+    fill_words((uint32_t *)const_cast<float *>(lights[l].shadowmap), 0x3f800000u, (size_t)N * N, t,
+               gridDim.x * blockDim.x);  // clear depth 1.0
+    if (t >= sc.ntri) return;
     const size_t slot = (size_t)blockIdx.y * (size_t)sc.ntri + (size_t)t;
     float clip[3][4];
     bool behind = false;
@@ -96,38 +116,17 @@ __global__ __launch_bounds__(256) void k_shadow_setup(DevScene sc, const DevLigh
     bcounts[slot] = 0;
 }
 
-// The triangle slot of every block of the block walk, one thread per block
-// (the search of k_raster_items, run for 64 blocks per wavefront so that the
-// dependent loads of many searches are in flight together).  Blocks beyond
-// `cap` are left to the walk's own search.
-__global__ __launch_bounds__(256) void k_block_slots(const uint64_t *__restrict__ offs,
-                                                     const uint32_t *__restrict__ chunk, size_t chunk_cap, int nslots,
-                                                     uint32_t *slots, size_t cap) {
-    const uint64_t total = offs[nslots];
-    const uint64_t n = total < cap ? total : cap;
-    const uint64_t nchunks = (total + 63) >> 6;
-    for (uint64_t k = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; k < n; k += (uint64_t)gridDim.x * blockDim.x) {
-        const uint64_t c = k >> 6;
-        int lo = c < chunk_cap ? (int)chunk[c] : 0;
-        int hi = (c + 1 < nchunks && c + 1 < chunk_cap) ? (int)chunk[c + 1] : nslots - 1;
-        while (lo < hi) {
-            const int mid = (lo + hi + 1) >> 1;
-            if (offs[mid] <= k) lo = mid;
-            else hi = mid - 1;
-        }
-        slots[k] = (uint32_t)lo;
-    }
-}
-
 // The large triangles of a walk, 8x8-pixel blocks of their bounding boxes, the
 // lanes a block's pixels (row-major).  A wavefront takes runs of consecutive
 // blocks (up to kBlockRun; run r by wavefront r % wavefronts, so that the runs
 // of covered blocks and of empty ones are dealt out evenly), and a triangle's
-// record is wave-uniform (its slot from k_block_slots, or the same search past
-// that table).  Each lane keeps its three edge values in FP64 and steps them
-// from block to block: every one is an integer below 2^53 (|A|, |B| <= 2^28, a
-// coordinate in 1/256 px below 2^22), so every sum is exact, the values are
-// those of edge_value in both of its forms, and the barycentrics are
+// record is wave-uniform: its slot is found in the offsets of up to 64 slots that
+// the lanes hold, read where a run begins or passes their end.  (A table of every
+// block's slot, filled by a launch of its own, took 10 to 23 us and left the walk
+// no faster: 534 us with it, 507 without.)  Each lane keeps its three edge values
+// in FP64 and steps them from block to block: every one is an integer below 2^53
+// (|A|, |B| <= 2^28, a coordinate in 1/256 px below 2^22), so every sum is exact,
+// the values are those of edge_value in both of its forms, and the barycentrics are
 // quot_f32(E, area) with the triangle's reciprocal: every fragment and its
 // barycentrics are those the pixel walk produces.  F provides Tri (a triangle's
 // wave-uniform data, the image size W x H among it), enter(slot, edges) that
@@ -142,7 +141,7 @@ __global__ __launch_bounds__(256) void k_block_slots(const uint64_t *__restrict_
 // instructions a block, in two forms (32-bit and FP64) whose arrays took 82
 // registers: 5 wavefronts per SIMD for a grid of 8, on equal shares of
 // consecutive blocks.  Five 1024^2 maps: 286 us before, 183; five 2048^2 maps:
-// 1024 us before, 534.  The load in the same stage as the atomic suits the depth
+// 1024 us before, 507.  The load in the same stage as the atomic suits the depth
 // maps (190 and 560 us with the G-buffer's stages); the G-buffer, fewer blocks
 // of longer triangles, waits for the load, so the atomic goes one block later
 // (1920x1080: 79 us without the load, 92 with it, 73 one block later; 3840x2160:
@@ -150,10 +149,15 @@ __global__ __launch_bounds__(256) void k_block_slots(const uint64_t *__restrict_
 
 constexpr int kBlockRun = 64;
 
+__device__ __forceinline__ uint64_t readlane_u64(uint64_t v, int lane) {
+    return ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(v >> 32), lane) << 32) |
+           (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)v, lane);
+}
+
 template <class F>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void k_raster_blocks(
     const int4 *__restrict__ recs, const uint64_t *__restrict__ offs, const uint32_t *__restrict__ chunk,
-    size_t chunk_cap, int nslots, const uint32_t *__restrict__ bslots, size_t bslots_cap, F f) {
+    size_t chunk_cap, int nslots, F f) {
     const uint64_t total = offs[nslots];
     const uint64_t nchunks = (total + 63) >> 6;
     const int lane = threadIdx.x & 63;
@@ -166,22 +170,30 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void k
     for (uint64_t r0 = wave * run; r0 < total; r0 += nwaves * run) {
         const uint64_t r1 = r0 + run < total ? r0 + run : total;
         uint64_t k = r0;
+        int lo = 0, known = 0;       // lane i holds the offset of slot lo + i, for `known` slots
+        uint64_t off = 0;
         while (k < r1) {  // the run's next triangle
-            int lo;
-            if (k < bslots_cap) {
-                lo = (int)bslots[k];
-            } else {
-                const uint64_t c = k >> 6;  // block k lies in chunk c (64 blocks per chunk)
-                lo = c < chunk_cap ? (int)chunk[c] : 0;
+            uint64_t m = __ballot(lane < known && off <= k);
+            if (m == 0 || m >> (known - 1) != 0) {  // not among the slots at hand
+                const uint64_t c = k >> 6;          // block k lies in chunk c (64 blocks per chunk)
+                const int first = c < chunk_cap ? (int)chunk[c] : 0;
                 int hi = (c + 1 < nchunks && c + 1 < chunk_cap) ? (int)chunk[c + 1] : nslots - 1;
-                while (lo < hi) {
-                    const int mid = (lo + hi + 1) >> 1;
-                    if (offs[mid] <= k) lo = mid;
-                    else hi = mid - 1;
+                lo = __builtin_amdgcn_readfirstlane(lo + known > first && known ? lo + known - 1 : first);
+                hi = __builtin_amdgcn_readfirstlane(hi);
+                while (hi - lo >= 63) {  // the last slot of [lo, hi] that starts at or before k, 64 probes at a time
+                    const int step = ((hi - lo) >> 6) + 1;
+                    const int p = lo + lane * step;
+                    const int top = 63 - __builtin_clzll(__ballot(p <= hi && offs[p <= hi ? p : hi] <= k));
+                    lo += top * step;
+                    hi = lo + step - 1 < hi ? lo + step - 1 : hi;
                 }
+                known = nslots - lo < 63 ? nslots - lo + 1 : 64;
+                off = offs[lo + (lane < known ? lane : 0)];
+                m = __ballot(lane < known && off <= k);
             }
-            const int slot = __builtin_amdgcn_readfirstlane(lo);
-            const uint64_t t0 = offs[slot], t1 = offs[slot + 1];
+            const int at = 63 - __builtin_clzll(m);
+            const int slot = lo + at;
+            const uint64_t t0 = readlane_u64(off, at), t1 = readlane_u64(off, at + 1);
             const uint32_t n = (uint32_t)((t1 < r1 ? t1 : r1) - k);  // its blocks in this run
             Edges e;
             load_edges(recs, (size_t)slot, e);
@@ -305,26 +317,21 @@ hipError_t launch_shadowmaps(const DevScene &sc, const DevLight *hlights, const 
     for (int j0 = 0; j0 < n; j0 += batch) {
         const int nb = n - j0 < batch ? n - j0 : batch;
         uint64_t packed = 0;
+        size_t texels = 0;
         for (int j = 0; j < nb; ++j) {
-            const DevLight &L = hlights[li[j0 + j]];
-            const size_t N = L.shadow_size;  // clear depth 1.0
-            if ((e = launch_fill_u32((uint32_t *)const_cast<float *>(L.shadowmap), 0x3f800000u, N * N, s)) !=
-                hipSuccess)
-                return e;
+            const size_t N = hlights[li[j0 + j]].shadow_size;
+            if (N * N > texels) texels = N * N;
             packed |= (uint64_t)(uint32_t)li[j0 + j] << (5 * j);
         }
+        const size_t nslots = (size_t)nb * (size_t)sc.ntri;
+        hipLaunchKernelGGL(k_shadow_setup, dim3(setup_blocks(sc.ntri, texels), nb), dim3(256), 0, s, sc, dlights,
+                           packed, rs.rec, rs.attr, rs.counts, rs.bcounts);
+        if ((e = hipGetLastError()) != hipSuccess) return e;
         if (sc.ntri > 0) {
-            const size_t nslots = (size_t)nb * (size_t)sc.ntri;
-            hipLaunchKernelGGL(k_shadow_setup, dim3((sc.ntri + 255) / 256, nb), dim3(256), 0, s, sc, dlights, packed,
-                               rs.rec, rs.attr, rs.counts, rs.bcounts);
-            if ((e = hipGetLastError()) != hipSuccess) return e;
             if ((e = raster_scan(rs, nslots, true, s)) != hipSuccess) return e;
             ShadowFrag f{rs.attr, dlights};
             hipLaunchKernelGGL(k_raster_items<ShadowFrag>, dim3(raster_grid<ShadowFrag, false>()), dim3(256), 0, s,
                                rs.rec, rs.offs, rs.chunk, rs.chunk_cap, (int)nslots, f);
-            if ((e = hipGetLastError()) != hipSuccess) return e;
-            hipLaunchKernelGGL(k_block_slots, dim3(kRasterBlocks), dim3(256), 0, s, rs.boffs, rs.bchunk, rs.chunk_cap,
-                               (int)nslots, rs.bslots, rs.bslots_cap);
             if ((e = hipGetLastError()) != hipSuccess) return e;
             ShadowBlockFrag fb{};
             fb.attr = rs.attr;
@@ -334,7 +341,7 @@ hipError_t launch_shadowmaps(const DevScene &sc, const DevLight *hlights, const 
                 fb.maps.size[li[j0 + j]] = (int)L.shadow_size;
             }
             hipLaunchKernelGGL(k_raster_blocks<ShadowBlockFrag>, dim3(kRasterBlocks), dim3(256), 0, s, rs.rec,
-                               rs.boffs, rs.bchunk, rs.chunk_cap, (int)nslots, rs.bslots, rs.bslots_cap, fb);
+                               rs.boffs, rs.bchunk, rs.chunk_cap, (int)nslots, fb);
             if ((e = hipGetLastError()) != hipSuccess) return e;
         }
         // the footprint layout of every map of the walk, one launch
@@ -392,8 +399,9 @@ struct CamMats {
 };
 
 __global__ __launch_bounds__(256) void k_gbuf_setup(DevScene sc, CamMats cm, int4 *rec, float4 *attr,
-                                                    uint32_t *counts, uint32_t *bcounts) {
+                                                    uint32_t *counts, uint32_t *bcounts, uint32_t *vis) {
     int t = blockIdx.x * blockDim.x + threadIdx.x;
+    fill_words(vis, ~0u, (size_t)cm.W * cm.H * 2, t, gridDim.x * blockDim.x);
     if (t >= sc.ntri) return;
     float clip[3][4];
     for (int v = 0; v < 3; ++v) {
@@ -486,16 +494,17 @@ struct GbufBlockFrag {
         int W, H;
     };
     struct Pending {
-        unsigned long long *d, key, seen;
+        unsigned long long key, seen;
+        uint32_t at;
         bool live;
     };
     __device__ Tri enter(int slot, const Edges &e) const { return Tri{attr[slot], 0xffffffffu - (uint32_t)e.user, W, H}; }
     __device__ Pending fetch(const Tri &, int px, int py, bool in) const {
         Pending p;
-        p.d = &vis[(size_t)(uint32_t)(py * W + px)];
+        p.at = (uint32_t)(py * W + px);
         p.key = p.seen = 0ull;
         p.live = in;
-        if (in) p.seen = vctk::seen(p.d);
+        if (in) p.seen = vctk::seen(&vis[p.at]);
         return p;
     }
     __device__ void depth(const Tri &t, const float l[3], Pending &p) const {
@@ -505,7 +514,7 @@ struct GbufBlockFrag {
         p.key = ((unsigned long long)__float_as_uint(z) << 32) | (unsigned long long)t.low;
     }
     __device__ void store(const Pending &p) const {
-        if (p.live && p.seen > p.key) atomicMin(p.d, p.key);
+        if (p.live && p.seen > p.key) atomicMin(&vis[p.at], p.key);
     }
 };
 
@@ -605,9 +614,7 @@ __global__ __launch_bounds__(256) void k_gbuf_resolve(DevScene sc, CamMats cm, c
 
 hipError_t launch_gbuffer(const DevScene &sc, const vct_camera &cam, uint64_t *vis, vct_gbuffer_texel *gbuf,
                           RasterScratch &rs, hipStream_t s) {
-    const size_t np = (size_t)cam.width * cam.height;
-    hipError_t e = launch_fill_u64(vis, ~0ull, np, s);
-    if (e != hipSuccess) return e;
+    hipError_t e;
     CamMats cm;
     // pv = projection * view, the matrix product phong.vert applies before model
     for (int c = 0; c < 4; ++c)
@@ -621,22 +628,19 @@ hipError_t launch_gbuffer(const DevScene &sc, const vct_camera &cam, uint64_t *v
     cm.W = cam.width;
     cm.H = cam.height;
     cm.cull = cam.cull_back;
+    const size_t nslots = (size_t)sc.ntri * 2;
+    hipLaunchKernelGGL(k_gbuf_setup, dim3(setup_blocks(sc.ntri, (size_t)cam.width * cam.height * 2)), dim3(256), 0, s,
+                       sc, cm, rs.rec, rs.attr, rs.counts, rs.bcounts, (uint32_t *)vis);
+    if ((e = hipGetLastError()) != hipSuccess) return e;
     if (sc.ntri > 0) {
-        const size_t nslots = (size_t)sc.ntri * 2;
-        hipLaunchKernelGGL(k_gbuf_setup, dim3((sc.ntri + 255) / 256), dim3(256), 0, s, sc, cm, rs.rec, rs.attr,
-                           rs.counts, rs.bcounts);
-        if ((e = hipGetLastError()) != hipSuccess) return e;
         if ((e = raster_scan(rs, nslots, true, s)) != hipSuccess) return e;
         GbufFrag f{rs.attr, (unsigned long long *)vis, cam.width};
         hipLaunchKernelGGL(k_raster_items<GbufFrag>, dim3(raster_grid<GbufFrag, false>()), dim3(256), 0, s, rs.rec, rs.offs,
                            rs.chunk, rs.chunk_cap, (int)nslots, f);
         if ((e = hipGetLastError()) != hipSuccess) return e;
-        hipLaunchKernelGGL(k_block_slots, dim3(kRasterBlocks), dim3(256), 0, s, rs.boffs, rs.bchunk, rs.chunk_cap,
-                           (int)nslots, rs.bslots, rs.bslots_cap);
-        if ((e = hipGetLastError()) != hipSuccess) return e;
         GbufBlockFrag fb{rs.attr, (unsigned long long *)vis, cam.width, cam.height};
         hipLaunchKernelGGL(k_raster_blocks<GbufBlockFrag>, dim3(kRasterBlocks), dim3(256), 0, s, rs.rec, rs.boffs,
-                           rs.bchunk, rs.chunk_cap, (int)nslots, rs.bslots, rs.bslots_cap, fb);
+                           rs.bchunk, rs.chunk_cap, (int)nslots, fb);
         if ((e = hipGetLastError()) != hipSuccess) return e;
     }
     dim3 grid((cam.width + 15) / 16, (cam.height + 15) / 16);

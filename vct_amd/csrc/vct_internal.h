@@ -145,8 +145,6 @@ struct RasterScratch {
     uint32_t *bcounts;
     uint64_t *boffs;
     uint32_t *bchunk;
-    uint32_t *bslots;   // the slot of each block, for the first bslots_cap blocks
-    size_t bslots_cap;
 };
 
 // The diffuse cones' step schedule.  Every diffuse cone of every pixel starts
@@ -201,13 +199,13 @@ NoAllocScratch noalloc_scratch(int device);    // nulls before the setup
 
 // ---- launch wrappers (return hipError_t of the last launch) ----------------
 hipError_t launch_fill_u32(uint32_t *p, uint32_t v, size_t n, hipStream_t s);
-hipError_t launch_fill_u64(uint64_t *p, uint64_t v, size_t n, hipStream_t s);
 // sums/maxes partials[0..n) (4 words each: sum, max, sum, sum) into the named stats fields
 hipError_t launch_reduce_stats(const uint32_t *partials, int n, uint32_t *sum0, uint32_t *max1, uint32_t *sum2,
                                hipStream_t s);
 
 // scan.hip: counts[0..n) -> offs[0..n] exclusive (offs[n] = total) and chunk
-// starts; with `blocks` the same for the block counts (bcounts -> boffs, bchunk)
+// starts; with `blocks` the same for the block counts (bcounts -> boffs, bchunk).
+// n >= 1.
 hipError_t raster_scan(RasterScratch &rs, size_t nslots, bool blocks, hipStream_t s);
 // the scan's tiles for nslots slots (rs.tsum holds 4 words per tile)
 size_t raster_scan_tiles(size_t nslots);
