@@ -2,11 +2,11 @@
 // src/Application.cpp:877-921) fused over three levels per launch.
 //
 // The reference dispatches one compute pass per level with a full barrier in
-// between, re-reading each level from memory.  Here one workgroup loads an
-// 8^3 region of the source level (two 4^3 bricks per axis, contiguous 512-byte
-// brick runs) into LDS and produces the 4^3, 2^3 and 1^3 blocks of the next
-// three levels from LDS, so level 0 -- the only large one -- is read exactly
-// once.  Each level is rounded to its storage format before the next one is
+// between, re-reading each level from memory.  Here a launch takes 8^3 regions
+// of the source level (two 4^3 bricks per axis, contiguous 1 KB brick runs) and
+// produces the 4^3, 2^3 and 1^3 blocks of the next three levels: a wavefront per
+// region where the source has one face (k_mip_regions), a workgroup where it has
+// six (k_mip_chain).  So level 0 -- the only large one -- is read exactly once.  Each level is rounded to its storage format before the next one is
 // filtered from it, exactly as a per-level pass over stored texels would be,
 // and the eight taps are summed in the reference's offset order, so the chain
 // is bit-identical to filtering level by level.
@@ -116,9 +116,8 @@ __device__ __forceinline__ void mip_step(const MipArgs &a, int cur_rt, int faces
 // faces w and w + 4, one texel per lane.  The face is wave-uniform, so the
 // child offsets of its near/far pairs are scalar values and only the texel's
 // base address is per lane.  Same taps, in the same order, as mip_step.
-template <bool ANISO, bool SRC6>
 __device__ __forceinline__ void mip_step8(const MipArgs &a, const float4 *in, float4 *out, int ox, int oy, int oz) {
-    constexpr int NF = ANISO ? 6 : 1;
+    constexpr int NF = 6;
     constexpr int cur = 8;
     const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int lane = threadIdx.x & 63;
@@ -126,51 +125,35 @@ __device__ __forceinline__ void mip_step8(const MipArgs &a, const float4 *in, fl
     const int base = ((2 * z) * cur + 2 * y) * cur + 2 * x;
     const LevelInfo &ol = a.out[0];
     for (int f = w; f < NF; f += 4) {
-        const float4 *c = in + (SRC6 ? f * 512 : 0) + base;
+        const float4 *c = in + f * 512 + base;
         float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-        if (!ANISO) {
+        const int ax = f >> 1, neg = f & 1;
+        // strides of the face's axis and of the two axes across it (oa, ob
+        // as in mip_step: y, z for x; x, z for y; x, y for z)
+        const int s_ax = ax == 0 ? 1 : (ax == 1 ? cur : cur * cur);
+        const int s_oa = ax == 0 ? cur : 1;
+        const int s_ob = ax == 2 ? cur : cur * cur;
+        const int near = neg ? s_ax : 0, far = neg ? 0 : s_ax;
 #pragma unroll
-            for (int o = 0; o < 8; ++o) {
-                const int dx = (o >> 2) & 1, dy = (o >> 1) & 1, dz = o & 1;
-                const float4 t = c[(dz * cur + dy) * cur + dx];
-                v.x = v.x + t.x;
-                v.y = v.y + t.y;
-                v.z = v.z + t.z;
-                v.w = v.w + t.w;
+        for (int pa = 0; pa < 2; ++pa)
+#pragma unroll
+            for (int pb = 0; pb < 2; ++pb) {
+                const int o = pa * s_oa + pb * s_ob;
+                const float4 pn = c[o + near];
+                const float4 pf = c[o + far];
+                const float t = 1.0f - pn.w;
+                v.x = v.x + (pn.x + t * pf.x);
+                v.y = v.y + (pn.y + t * pf.y);
+                v.z = v.z + (pn.z + t * pf.z);
+                v.w = v.w + (pn.w + t * pf.w);
             }
-            v.x = v.x * 0.125f;
-            v.y = v.y * 0.125f;
-            v.z = v.z * 0.125f;
-            v.w = v.w * 0.125f;
-        } else {
-            const int ax = f >> 1, neg = f & 1;
-            // strides of the face's axis and of the two axes across it (oa, ob
-            // as in mip_step: y, z for x; x, z for y; x, y for z)
-            const int s_ax = ax == 0 ? 1 : (ax == 1 ? cur : cur * cur);
-            const int s_oa = ax == 0 ? cur : 1;
-            const int s_ob = ax == 2 ? cur : cur * cur;
-            const int near = neg ? s_ax : 0, far = neg ? 0 : s_ax;
-#pragma unroll
-            for (int pa = 0; pa < 2; ++pa)
-#pragma unroll
-                for (int pb = 0; pb < 2; ++pb) {
-                    const int o = pa * s_oa + pb * s_ob;
-                    const float4 pn = c[o + near];
-                    const float4 pf = c[o + far];
-                    const float t = 1.0f - pn.w;
-                    v.x = v.x + (pn.x + t * pf.x);
-                    v.y = v.y + (pn.y + t * pf.y);
-                    v.z = v.z + (pn.z + t * pf.z);
-                    v.w = v.w + (pn.w + t * pf.w);
-                }
-            v.x = v.x * 0.25f;
-            v.y = v.y * 0.25f;
-            v.z = v.z * 0.25f;
-            v.w = v.w * 0.25f;
-        }
+        v.x = v.x * 0.25f;
+        v.y = v.y * 0.25f;
+        v.z = v.z * 0.25f;
+        v.w = v.w * 0.25f;
         v = round_stage(v, a.fp32);
         out[f * 64 + lane] = v;
-        store_stage_texel(a.pyr, ol, (ox >> 1) + x, (oy >> 1) + y, (oz >> 1) + z, NF == 6 ? f : 0, v);
+        store_stage_texel(a.pyr, ol, (ox >> 1) + x, (oy >> 1) + y, (oz >> 1) + z, f, v);
     }
 }
 
@@ -229,8 +212,8 @@ __global__ __launch_bounds__(256) void k_mip_chain(MipArgs a) {
         }
     }
     __syncthreads();
-    if (R == 8) {  // the three steps with their sizes known at compile time
-        mip_step8<ANISO, SRC6>(a, &bufA[0][0], &bufB[0][0], ox, oy, oz);
+    if (SRC6 && R == 8) {  // the three steps with their sizes known at compile time
+        mip_step8(a, &bufA[0][0], &bufB[0][0], ox, oy, oz);
         if (a.nout > 1) {
             __syncthreads();
             mip_step<ANISO, 4>(a, 4, NF, &bufB[0][0], 64, &bufA[0][0], 8, 1, ox, oy, oz);
@@ -257,6 +240,156 @@ __global__ __launch_bounds__(256) void k_mip_chain(MipArgs a) {
         in_stride = out_stride;
         cur = d;
         faces = NF;
+    }
+}
+
+// One wavefront per 8^3 region of a source with one face, one output texel per
+// lane: the lane loads its eight children (four pair elements, or eight fp32
+// texels) and filters all its faces in registers; the two smaller steps go
+// through LDS within the wavefront.  Same taps, in the same order, as mip_step.
+//
+// What bounds it: memory (1 KB read per brick that is not zero, 16 bytes written
+// per texel and face).  With a workgroup per region, the children in LDS and a
+// barrier before each step, three of four wavefronts waited in the isotropic
+// steps and a CU had 8 regions in flight: the chain of 512^3 461 us, now 308;
+// 256^3 with six faces 113, 110 (both at 3.3 TB/s beside the albedo chain); 128^3
+// 13.8, 9.4.  Not storing zeros over zeros again (a record per region) gained
+// nothing: two thirds of the regions of a 256^3 scene hold something.
+template <bool ANISO, int CUR>
+__device__ __forceinline__ float4 mip_wave_texel(const float4 *in, int f, int x, int y, int z) {
+    const float4 *c = in + ((2 * z) * CUR + 2 * y) * CUR + 2 * x;
+    float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (!ANISO) {
+#pragma unroll
+        for (int o = 0; o < 8; ++o) {
+            const float4 t = c[((o & 1) * CUR + ((o >> 1) & 1)) * CUR + (o >> 2)];
+            v.x = v.x + t.x;
+            v.y = v.y + t.y;
+            v.z = v.z + t.z;
+            v.w = v.w + t.w;
+        }
+        return make_float4(v.x * 0.125f, v.y * 0.125f, v.z * 0.125f, v.w * 0.125f);
+    }
+    const int ax = f >> 1, neg = f & 1;
+    const int s_ax = ax == 0 ? 1 : (ax == 1 ? CUR : CUR * CUR);  // strides as in mip_step8
+    const int s_oa = ax == 0 ? CUR : 1;
+    const int s_ob = ax == 2 ? CUR : CUR * CUR;
+    const int near = neg ? s_ax : 0, far = neg ? 0 : s_ax;
+#pragma unroll
+    for (int p = 0; p < 4; ++p) {
+        const int o = (p >> 1) * s_oa + (p & 1) * s_ob;
+        const float4 pn = c[o + near];
+        const float4 pf = c[o + far];
+        const float t = 1.0f - pn.w;
+        v.x = v.x + (pn.x + t * pf.x);
+        v.y = v.y + (pn.y + t * pf.y);
+        v.z = v.z + (pn.z + t * pf.z);
+        v.w = v.w + (pn.w + t * pf.w);
+    }
+    return make_float4(v.x * 0.25f, v.y * 0.25f, v.z * 0.25f, v.w * 0.25f);
+}
+
+template <bool ANISO, bool FP32>
+__global__ __launch_bounds__(256) void k_mip_regions(MipArgs a) {
+    constexpr int NF = ANISO ? 6 : 1;
+    __shared__ float4 buf1[4][NF][64], buf2[4][NF][8];
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const uint32_t nreg = (uint32_t)a.src.size >> 3;  // a power of two, as every level's size
+    const int lg = __builtin_ctz(nreg);
+    // XCD-aware order: workgroup b runs on XCD b % 8, so give each XCD a
+    // contiguous run of regions; x-neighbours then share an L2 and run at
+    // about the same time, which merges the two halves of the pair elements
+    // on a region's x boundary in one L2 line before it is written back.
+    const uint32_t nblk = gridDim.x;
+    const uint32_t b = (nblk & 7u) == 0 ? (blockIdx.x & 7u) * (nblk >> 3) + (blockIdx.x >> 3) : blockIdx.x;
+    const uint32_t r = b * 4u + (uint32_t)w;
+    if (r >= nreg * nreg * nreg) return;  // no barrier below
+    const int ox = (int)(r & (nreg - 1)) * 8, oy = (int)((r >> lg) & (nreg - 1)) * 8, oz = (int)(r >> (2 * lg)) * 8;
+    const int X = lane & 3, Y = (lane >> 2) & 3, Z = lane >> 4;
+    const int x = ox + 2 * X, y = oy + 2 * Y, z = oz + 2 * Z;  // the lane's children lie in one brick
+    const bool zero = src_zero(a, x, y, z);
+    const bool none = __ballot(!zero) == 0;
+    float4 c[8];  // child (dx, dy, dz) = bits (2, 1, 0)
+#pragma unroll
+    for (int o = 0; o < 8; ++o) c[o] = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (!zero) {
+        const char *p = a.pyr + a.src.stage + (size_t)elem_index(a.src, x, y, z, 0) * 16;
+        if (FP32) {
+#pragma unroll
+            for (int o = 0; o < 8; ++o)
+                c[o] = *(const float4 *)(p + ((o >> 2) + ((o >> 1) & 1) * 4 + (o & 1) * 16) * 16);
+        } else {  // the element of an even x holds texels x and x + 1
+#pragma unroll
+            for (int o = 0; o < 4; ++o) {
+                const uint4 e = *(const uint4 *)(p + (((o >> 1) & 1) * 4 + (o & 1) * 16) * 16);
+                c[o] = unpack_h4(e.x, e.y);
+                c[4 + o] = unpack_h4(e.z, e.w);
+            }
+        }
+    }
+    const LevelInfo &ol = a.out[0];
+    const int gx = (ox >> 1) + X, gy = (oy >> 1) + Y, gz = (oz >> 1) + Z;  // a region's outputs are one brick
+    char *const q = a.pyr + ol.stage + (size_t)elem_index(ol, gx, gy, gz, 0) * 16;
+    const uint32_t ql = ol.stage + elem_index(ol, gx - 1, gy, gz, 0) * 16u;  // wraps below 0 at gx = 0
+#pragma unroll
+    for (int f = 0; f < NF; ++f) {
+        float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (none) {
+            // zeros filter to +0
+        } else if (!ANISO) {
+            // BOX2 offsets in filterRadiance.comp order: (0,0,0),(0,0,1),(0,1,0),(0,1,1),(1,0,0),...
+#pragma unroll
+            for (int o = 0; o < 8; ++o) {
+                v.x = v.x + c[o].x;
+                v.y = v.y + c[o].y;
+                v.z = v.z + c[o].z;
+                v.w = v.w + c[o].w;
+            }
+            v = make_float4(v.x * 0.125f, v.y * 0.125f, v.z * 0.125f, v.w * 0.125f);
+        } else {
+            const int ax = f >> 1, neg = f & 1;
+            const int b_ax = 4 >> ax;                             // the bits of c's index: the face's axis
+            const int b_oa = ax == 0 ? 2 : 4, b_ob = ax == 2 ? 2 : 1;  // and the two across it
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const int o = (k >> 1 ? b_oa : 0) | (k & 1 ? b_ob : 0);
+                const float4 pn = c[o | (neg ? b_ax : 0)], pf = c[o | (neg ? 0 : b_ax)];
+                const float t = 1.0f - pn.w;
+                v.x = v.x + (pn.x + t * pf.x);
+                v.y = v.y + (pn.y + t * pf.y);
+                v.z = v.z + (pn.z + t * pf.z);
+                v.w = v.w + (pn.w + t * pf.w);
+            }
+            v = make_float4(v.x * 0.25f, v.y * 0.25f, v.z * 0.25f, v.w * 0.25f);
+        }
+        v = round_stage(v, FP32);
+        if (!none) buf1[w][f][lane] = v;
+        if (FP32) {
+            *(float4 *)(q + f * 1024) = v;
+        } else {
+            // the lane's element: its texel and the next one in x, which the next
+            // region stores for the last
+            const uint2 h = pack_h4(v);
+            const uint2 n = make_uint2(__shfl_down(h.x, 1, 64), __shfl_down(h.y, 1, 64));
+            if (X < 3) *(uint4 *)(q + f * 1024) = make_uint4(h.x, h.y, n.x, n.y);
+            else *(uint2 *)(q + f * 1024) = h;
+            if (X == 0) *(uint2 *)(a.pyr + (uint32_t)(ql + f * 1024u) + 8) = h;
+        }
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    if (a.nout > 1 && lane < 8 * NF) {
+        const int f = lane >> 3, vi = lane & 7;
+        float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (!none) v = round_stage(mip_wave_texel<ANISO, 4>(buf1[w][f], f, vi & 1, (vi >> 1) & 1, vi >> 2), FP32);
+        buf2[w][f][vi] = v;
+        store_stage_texel(a.pyr, a.out[1], (ox >> 2) + (vi & 1), (oy >> 2) + ((vi >> 1) & 1), (oz >> 2) + (vi >> 2), f, v);
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    if (a.nout > 2 && lane < NF) {
+        const float4 v = round_stage(mip_wave_texel<ANISO, 2>(buf2[w][lane], lane, 0, 0, 0), FP32);
+        store_stage_texel(a.pyr, a.out[2], ox >> 3, oy >> 3, oz >> 3, lane, v);
     }
 }
 
@@ -480,7 +613,14 @@ hipError_t launch_mip(const PyrDesc &pyr, hipStream_t s) {
         a.zero0 = src == 0 ? pyr.zero0 : nullptr;
         const int nreg = S.size / R;
         dim3 grid((unsigned)(nreg * nreg * nreg));
-        if (pyr.aniso && S.nfaces == 6) hipLaunchKernelGGL((k_mip_chain<true, true>), grid, dim3(256), 0, s, a);
+        const dim3 wgrid((grid.x + 3) / 4);  // a wavefront per region
+        if (R == 8 && S.nfaces == 1 && pyr.aniso) {
+            if (fp32) hipLaunchKernelGGL((k_mip_regions<true, true>), wgrid, dim3(256), 0, s, a);
+            else hipLaunchKernelGGL((k_mip_regions<true, false>), wgrid, dim3(256), 0, s, a);
+        } else if (R == 8 && S.nfaces == 1) {
+            if (fp32) hipLaunchKernelGGL((k_mip_regions<false, true>), wgrid, dim3(256), 0, s, a);
+            else hipLaunchKernelGGL((k_mip_regions<false, false>), wgrid, dim3(256), 0, s, a);
+        } else if (pyr.aniso && S.nfaces == 6) hipLaunchKernelGGL((k_mip_chain<true, true>), grid, dim3(256), 0, s, a);
         else if (pyr.aniso) hipLaunchKernelGGL((k_mip_chain<true, false>), grid, dim3(256), 0, s, a);
         else hipLaunchKernelGGL((k_mip_chain<false, false>), grid, dim3(256), 0, s, a);
         hipError_t e = hipGetLastError();

@@ -179,23 +179,32 @@ __device__ __forceinline__ uint2 inject_texel_h(uint32_t a32, bool lit, float op
                       (uint32_t)h16[(a32 >> 16) & 0xffu] | (na_h << 16));
 }
 
-// One wavefront per 4^3 brick, one voxel per lane in the brick's element
-// order (lane = (x&3) | (y&3) << 2 | (z&3) << 4, the same for the bricked
-// albedo grid and for level 0), so albedo reads are one 256-byte run and each
-// level-0 store is one contiguous run of the brick's elements: 1 KB of fp16
+// One wavefront per run of 2^lgrun 4^3 bricks along x, one voxel per lane in the
+// brick's element order (lane = (x&3) | (y&3) << 2 | (z&3) << 4, the same for the
+// bricked albedo grid and for level 0), so albedo reads are one 256-byte run and
+// each level-0 store is one contiguous run of the brick's elements: 1 KB of fp16
 // pairs or fp32 texels.  An fp16 pair element x holds texels x and x+1: the
-// second comes from the next lane, or for the last voxel of a brick row from
-// that voxel's own inputs in the next brick (texel dim is the zero border).
-// The grid strides over the bricks with a fixed number of workgroups, each of
+// second comes from the next lane, or for the last voxel of a brick row from the
+// next brick's words, which the wavefront reads one brick ahead in any case
+// (texel dim is the zero border).
+// The grid strides over the runs with a fixed number of workgroups, each of
 // which reduces its statistics in LDS and writes one partial.
 // The opacity rewrite of the albedo word (rewrite = 1) races with the read of
-// that word by the neighbouring brick's wavefront; either value gives the same
+// that word by the neighbouring run's wavefront; either value gives the same
 // texel, except when the opacity rounds to an alpha byte of 0 -- then the
 // launcher passes rewrite = 0 and rewrites in a pass of its own afterwards.
+//
+// What bounds it: memory (the albedo words, and 1.25 KB written per brick that is
+// not empty).  With a wavefront per brick in turn, each line of the linear lit
+// mask (32 bricks) went to all eight XCDs, and every brick read the mask and its
+// neighbour's words: 2.7 GB from memory for 0.7 GB of albedo and mask at 512^3.
+// A run keeps a line within its workgroup, a mask byte is read for a voxel that
+// holds something, and an empty brick in front of an empty one ends after the
+// comparison: 512^3 711 us before, 480; 256^3 93, 83; 128^3 12.2, 11.2.
 template <int FMT, bool TEMPORAL>
 __global__ __launch_bounds__(256) void k_normalize_inject(uint32_t *albedo, const uint8_t *__restrict__ litmask,
                                                           int dim, LevelInfo L0, float opacity, float decay,
-                                                          int rewrite, char *pyr, uint8_t *zero0,
+                                                          int rewrite, int lgrun, char *pyr, uint8_t *zero0,
                                                           uint32_t *partials) {
     const float mw = 1.0f - decay;  // the mix weight of this frame's value
     const float pw = 1.0f - mw;     // and of the previous one, as GLSL mix computes it
@@ -216,76 +225,95 @@ __global__ __launch_bounds__(256) void k_normalize_inject(uint32_t *albedo, cons
     const int lgnb = __builtin_ctz((unsigned)nb);
     const int lane = threadIdx.x & 63;
     const int vx = lane & 3, vy = (lane >> 2) & 3, vz = lane >> 4;
+    const int run = 1 << lgrun;
     uint32_t uniq = 0, maxf = 0, lit_count = 0;
-    for (uint32_t b = blockIdx.x * 4u + (threadIdx.x >> 6); b < nbricks; b += gridDim.x * 4u) {
+    for (uint32_t r = blockIdx.x * 4u + (threadIdx.x >> 6); r < nbricks >> lgrun; r += gridDim.x * 4u) {
         // nb = dim / 4 is a power of two (dim is one): shifts and masks
-        const int bx = (int)(b & (uint32_t)(nb - 1)), by = (int)((b >> lgnb) & (uint32_t)(nb - 1)),
-                  bz = (int)(b >> (2 * lgnb));
-        const int x = bx * 4 + vx, y = by * 4 + vy, z = bz * 4 + vz;
-        const size_t gi = ((size_t)b << 6) + (size_t)lane;  // grid_index(x, y, z)
-        const size_t li = ((size_t)z * dim + y) * dim + x;   // the lit mask is linear
-        const uint32_t a32 = albedo[gi];
-        const bool lit = litmask[li] != 0;
-        char *elem = pyr + L0.stage + (size_t)elem_index(L0, x, y, z, 0) * 16;
-        // the brick's elements already hold +0 (wave-uniform)
-        const uint32_t z0 = zero0 != nullptr ? (uint32_t)zero0[b] : 0u;  // PyrDesc::zero0 bits
-        const bool was0 = (z0 & 1u) != 0u;
-        float4 prev = make_float4(0.f, 0.f, 0.f, 0.f), prev1 = prev;
-        if (TEMPORAL && !was0) {  // this element as stored last frame (texels x, x+1 for fp16 pairs)
-            const uint4 e = *(const uint4 *)elem;
-            if (FMT == 1) {
-                prev = make_float4(__uint_as_float(e.x), __uint_as_float(e.y), __uint_as_float(e.z),
-                                   __uint_as_float(e.w));
-            } else {
-                prev = unpack_h4(e.x, e.y);
-                prev1 = unpack_h4(e.z, e.w);
+        const uint32_t b0 = __builtin_amdgcn_readfirstlane(r << lgrun);
+        const int bx0 = (int)(b0 & (uint32_t)(nb - 1)), by = (int)((b0 >> lgnb) & (uint32_t)(nb - 1)),
+                  bz = (int)(b0 >> (2 * lgnb));
+        const int y = by * 4 + vy, z = bz * 4 + vz;
+        uint32_t *words = albedo + ((size_t)b0 << 6) + lane;  // grid_index(x, y, z)
+        const uint8_t *lits = litmask + ((size_t)z * dim + y) * dim + bx0 * 4 + vx;  // the lit mask is linear
+        char *elem = pyr + L0.stage + (size_t)elem_index(L0, bx0 * 4 + vx, y, z, 0) * 16;
+        // lane i: brick b0 + i's zero record (PyrDesc::zero0 bits), as it was and as it is
+        const uint32_t zr = zero0 != nullptr && lane < run ? (uint32_t)zero0[b0 + lane] : 0u;
+        uint32_t zw = zr;
+        uint32_t a32 = words[0], ahead = bx0 + 1 < nb ? words[64] : 0u;
+        for (int i = 0; i < run; ++i, words += 64, lits += 4, elem += (size_t)L0.sx * 16) {
+            const int x = (bx0 + i) * 4 + vx;
+            const uint32_t cur = a32, next = ahead;
+            a32 = next;
+            ahead = i + 1 < run && bx0 + i + 2 < nb ? words[128] : 0u;
+            // the brick's elements already hold +0 (wave-uniform)
+            const uint32_t z0 = __builtin_amdgcn_readlane(zr, i);
+            const bool was0 = (z0 & 1u) != 0u;
+            // no voxel of the brick and, for the pair elements, of the next one's first column holds anything
+            const bool empty =
+                !TEMPORAL && __ballot((cur >> 24) != 0u || (FMT == 0 && vx == 0 && (next >> 24) != 0u)) == 0;
+            bool now0 = true;
+            uint32_t nw = cur;
+            if (!empty) {
+                const bool lit = (TEMPORAL || (cur >> 24) != 0u) && *lits != 0;
+                float4 prev = make_float4(0.f, 0.f, 0.f, 0.f), prev1 = prev;
+                if (TEMPORAL && !was0) {  // this element as stored last frame (texels x, x+1 for fp16 pairs)
+                    const uint4 e = *(const uint4 *)elem;
+                    if (FMT == 1) {
+                        prev = make_float4(__uint_as_float(e.x), __uint_as_float(e.y), __uint_as_float(e.z),
+                                           __uint_as_float(e.w));
+                    } else {
+                        prev = unpack_h4(e.x, e.y);
+                        prev1 = unpack_h4(e.z, e.w);
+                    }
+                }
+                constexpr bool LUT = FMT == 0 && !TEMPORAL;
+                float4 c = make_float4(0.f, 0.f, 0.f, 0.f);
+                uint2 h = make_uint2(0u, 0u);
+                if (LUT) h = inject_texel_h(cur, lit, opacity, op_b, op_h, h16, &nw);
+                else c = inject_texel<TEMPORAL>(cur, lit, opacity, prev, mw, pw, &nw);
+                if ((cur >> 24) != 0u) {
+                    uniq += 1;
+                    const uint32_t mf = mf8[cur >> 24];
+                    maxf = mf > maxf ? mf : maxf;
+                    lit_count += lit ? 1u : 0u;
+                }
+                if (rewrite && nw != cur) *words = nw;
+                if (FMT == 1) {
+                    now0 = __ballot((__float_as_uint(c.x) | __float_as_uint(c.y) | __float_as_uint(c.z) |
+                                     __float_as_uint(c.w)) != 0u) == 0;
+                    if (!(now0 && was0)) *(float4 *)elem = c;  // an all-zero brick over zeros is not rewritten
+                } else {
+                    if (!LUT) h = pack_h4(c);
+                    uint2 h1 = make_uint2(__shfl_down(h.x, 1, 64), __shfl_down(h.y, 1, 64));  // texel x+1 in lane + 1
+                    const uint32_t a1 = __shfl(next, lane & ~3, 64);  // voxel x+1 opens the next brick
+                    if (vx == 3) {
+                        h1 = make_uint2(0u, 0u);  // texel dim: the border
+                        if (x + 1 < dim) {
+                            const bool lit1 = (TEMPORAL || (a1 >> 24) != 0u) && lits[1] != 0;
+                            uint32_t nw1;
+                            if (LUT) h1 = inject_texel_h(a1, lit1, opacity, op_b, op_h, h16, &nw1);
+                            else h1 = pack_h4(inject_texel<TEMPORAL>(a1, lit1, opacity, prev1, mw, pw, &nw1));
+                        }
+                    }
+                    now0 = __ballot((h.x | h.y | h1.x | h1.y) != 0u) == 0;
+                    if (!(now0 && was0)) {  // an all-zero brick over zeros is not rewritten
+                        *(uint4 *)elem = make_uint4(h.x, h.y, h1.x, h1.y);
+                        if (x == 0)  // texel 0 is also the second half of element -1, in the border brick
+                            *(uint2 *)(pyr + (uint32_t)(L0.stage + elem_index(L0, -1, y, z, 0) * 16u) + 8) = h;
+                    }
+                }
+            } else if (!was0) {
+                *(uint4 *)elem = make_uint4(0u, 0u, 0u, 0u);
+                if (FMT == 0 && x == 0)
+                    *(uint2 *)(pyr + (uint32_t)(L0.stage + elem_index(L0, -1, y, z, 0) * 16u) + 8) = make_uint2(0u, 0u);
             }
+            // every albedo word of the brick is 0 (a word that is 0 stays 0 under
+            // any later opacity rewrite); and was 0 as the voxelizer left it
+            const uint32_t z1 =
+                (now0 ? 1u : 0u) | (__ballot(nw != 0u) == 0 ? 2u : 0u) | (__ballot(cur != 0u) == 0 ? 4u : 0u);
+            if (lane == i) zw = z1;
         }
-        uint32_t nw;
-        constexpr bool LUT = FMT == 0 && !TEMPORAL;
-        float4 r = make_float4(0.f, 0.f, 0.f, 0.f);
-        uint2 h = make_uint2(0u, 0u);
-        if (LUT) h = inject_texel_h(a32, lit, opacity, op_b, op_h, h16, &nw);
-        else r = inject_texel<TEMPORAL>(a32, lit, opacity, prev, mw, pw, &nw);
-        if ((a32 >> 24) != 0u) {
-            uniq += 1;
-            const uint32_t mf = mf8[a32 >> 24];
-            maxf = mf > maxf ? mf : maxf;
-            lit_count += lit ? 1u : 0u;
-        }
-        if (rewrite && nw != a32) albedo[gi] = nw;
-        // every albedo word of the brick is 0 (a word that is 0 stays 0 under
-        // any later opacity rewrite); and was 0 as the voxelizer left it
-        const uint32_t za = (__ballot(nw != 0u) == 0 ? 2u : 0u) | (__ballot(a32 != 0u) == 0 ? 4u : 0u);
-        if (FMT == 1) {
-            const bool nz = (__float_as_uint(r.x) | __float_as_uint(r.y) | __float_as_uint(r.z) |
-                             __float_as_uint(r.w)) != 0u;
-            const bool now0 = __ballot(nz) == 0;
-            if (!(now0 && was0)) *(float4 *)elem = r;  // an all-zero brick over zeros is not rewritten
-            const uint32_t z1 = (now0 ? 1u : 0u) | za;
-            if (zero0 != nullptr && lane == 0 && z1 != z0) zero0[b] = (uint8_t)z1;
-            continue;
-        }
-        if (!LUT) h = pack_h4(r);
-        uint2 h1 = make_uint2(__shfl_down(h.x, 1, 64), __shfl_down(h.y, 1, 64));  // texel x+1 in lane + 1
-        if (vx == 3) {
-            h1 = make_uint2(0u, 0u);  // texel dim: the border
-            if (x + 1 < dim) {        // voxel x+1 opens brick b+1 along x
-                const uint32_t a1 = albedo[gi + 64 - 3];
-                const bool lit1 = litmask[li + 1] != 0;
-                uint32_t nw1;
-                if (LUT) h1 = inject_texel_h(a1, lit1, opacity, op_b, op_h, h16, &nw1);
-                else h1 = pack_h4(inject_texel<TEMPORAL>(a1, lit1, opacity, prev1, mw, pw, &nw1));
-            }
-        }
-        const bool now0 = __ballot((h.x | h.y | h1.x | h1.y) != 0u) == 0;
-        if (!(now0 && was0)) {  // an all-zero brick over zeros is not rewritten
-            *(uint4 *)elem = make_uint4(h.x, h.y, h1.x, h1.y);
-            if (x == 0)  // texel 0 is also the second half of element -1, in the border brick
-                *(uint2 *)(pyr + (uint32_t)(L0.stage + elem_index(L0, -1, y, z, 0) * 16u) + 8) = h;
-        }
-        const uint32_t z1 = (now0 ? 1u : 0u) | za;
-        if (zero0 != nullptr && lane == 0 && z1 != z0) zero0[b] = (uint8_t)z1;
+        if (zero0 != nullptr && lane < run && zw != zr) zero0[b0 + lane] = (uint8_t)zw;
     }
     block_partial(uniq, maxf, lit_count, 0u, partials);
 }
@@ -306,14 +334,18 @@ hipError_t launch_normalize_inject(uint32_t *albedo, const uint8_t *litmask, int
                                    hipStream_t s) {
     const LevelInfo &L0 = pyr.lv[0];
     const size_t nbricks = (size_t)L0.nb * L0.nb * L0.nb;
-    size_t blocks = (nbricks + 3) / 4;
+    // runs of up to 16 bricks within a row of the grid, as long as they leave the
+    // chip its 8192 wavefronts
+    int lgrun = 0;
+    while (lgrun < 4 && (2 << lgrun) <= L0.nb && nbricks >> (lgrun + 1) >= 8192) ++lgrun;
+    size_t blocks = ((nbricks >> lgrun) + 3) / 4;
     if (blocks > (size_t)kStatPartials) blocks = kStatPartials;
     dim3 grid((unsigned)blocks);
     // pack_unorm4x8 rounds opacity * 255: below 0.5 the rewritten alpha byte is 0
     const int rewrite = (opacity > 0.0f && opacity * 255.0f < 0.5f) ? 0 : 1;
 #define VCT_INJECT_LAUNCH(F, T)                                                                                     \
     hipLaunchKernelGGL((k_normalize_inject<F, T>), grid, dim3(256), 0, s, albedo, litmask, dim, L0, opacity, decay, \
-                       rewrite, pyr.pyr, pyr.zero0, partials)
+                       rewrite, lgrun, pyr.pyr, pyr.zero0, partials)
     if (L0.fmt == 1 && temporal) VCT_INJECT_LAUNCH(1, true);
     else if (L0.fmt == 1) VCT_INJECT_LAUNCH(1, false);
     else if (temporal) VCT_INJECT_LAUNCH(0, true);
