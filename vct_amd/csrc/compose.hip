@@ -120,10 +120,10 @@ __global__ __launch_bounds__(256) void k_compose(ComposeArgs a) {
                 ls[c] = (((ksp * att) * Lt.color[c]) * Lt.intensity) * alb[c];
             }
         }
-        if (Lt.shadow_caster && Lt.shadowquad) {
+        if (Lt.shadow_caster && Lt.shadowpad) {
             float w4[4] = {P[0], P[1], P[2], 1.0f}, lsp[4];
             mat4_vec4(Lt.ls, w4, lsp);
-            const float sf = 1.0f - calc_shadow_factor(lsp, Lt.shadowquad, (int)Lt.shadow_size);
+            const float sf = 1.0f - calc_shadow_factor(lsp, Lt.shadowpad, (int)Lt.shadow_size);
             for (int c = 0; c < 3; ++c) {
                 ld[c] = ld[c] * sf;
                 ls[c] = ls[c] * sf;

@@ -62,7 +62,7 @@ struct vct_ctx {
     // lights
     std::vector<vct_light> lights;
     std::vector<float *> d_shadow;
-    std::vector<float4 *> d_shadowq;  // footprint layout of each map (DevLight::shadowquad)
+    std::vector<float *> d_shadowp;  // padded copy of each map (DevLight::shadowpad)
     std::vector<DevLight> hlights;
     DevLight *d_lights = nullptr;
     // voxel grids
@@ -428,7 +428,7 @@ void vct_destroy(vct_ctx *c) {
     dfree(c->d_nmat);
     free_xf_ring(c);
     for (auto &p : c->d_shadow) dfree(p);
-    for (auto &p : c->d_shadowq) dfree(p);
+    for (auto &p : c->d_shadowp) dfree(p);
     dfree(c->d_lights);
     dfree(c->rs.rec);
     dfree(c->rs.attr);
@@ -720,28 +720,28 @@ int vct_set_lights(vct_ctx *c, const vct_light *lights, int n) {
     HIPCHK(c, hipStreamSynchronize(c->stream));
     // keep shadow maps whose size is unchanged (rebuilt per frame by vct_shadowmap(s))
     std::vector<float *> maps(n, nullptr);
-    std::vector<float4 *> quads(n, nullptr);
+    std::vector<float *> pads(n, nullptr);
     for (int i = 0; i < n; ++i) {
         const bool want = lights[i].shadow_caster != 0;
         if (want && i < (int)c->d_shadow.size() && c->d_shadow[i] && i < (int)c->lights.size() &&
             c->lights[i].shadow_caster && c->lights[i].shadow_size == lights[i].shadow_size) {
             maps[i] = c->d_shadow[i];
-            quads[i] = c->d_shadowq[i];
+            pads[i] = c->d_shadowp[i];
             c->d_shadow[i] = nullptr;
-            c->d_shadowq[i] = nullptr;
+            c->d_shadowp[i] = nullptr;
         } else if (want) {
             const size_t N = lights[i].shadow_size;
             HIPCHK(c, dalloc(&maps[i], N * N * 4));
-            HIPCHK(c, dalloc(&quads[i], (N + 1) * (N + 1) * 16));
+            HIPCHK(c, dalloc(&pads[i], (N + 2 * kShadowPad) * (N + 2 * kShadowPad) * 4));
             if (launch_fill_u32((uint32_t *)maps[i], 0x3f800000u, N * N, c->stream) != hipSuccess ||
-                launch_shadow_quads(maps[i], (int)N, quads[i], c->stream) != hipSuccess)
+                launch_shadow_pad(maps[i], (int)N, pads[i], c->stream) != hipSuccess)
                 return fail(c, VCT_ERR_HIP, "shadow map clear failed");
         }
     }
     for (auto &p : c->d_shadow) dfree(p);
-    for (auto &p : c->d_shadowq) dfree(p);
+    for (auto &p : c->d_shadowp) dfree(p);
     c->d_shadow = maps;
-    c->d_shadowq = quads;
+    c->d_shadowp = pads;
     c->lights.assign(lights, lights + n);
     c->hlights.resize(n);
     for (int i = 0; i < n; ++i) {
@@ -760,7 +760,7 @@ int vct_set_lights(vct_ctx *c, const vct_light *lights, int n) {
         memcpy(d.ls, L.ls, 64);
         memcpy(d.ls_inverse, L.ls_inverse, 64);
         d.shadowmap = maps[i];
-        d.shadowquad = quads[i];
+        d.shadowpad = pads[i];
     }
     dfree(c->d_lights);
     if (n) {
@@ -1321,7 +1321,7 @@ int vct_upload(vct_ctx *c, int what, int level, const void *host, size_t bytes) 
     case VCT_BUF_LITMASK: dst = c->d_litmask; break;
     case VCT_BUF_SHADOWMAP: {
         HIPCHK(c, hipMemcpyAsync(c->d_shadow[level], host, bytes, hipMemcpyHostToDevice, c->stream));
-        LAUNCHCHK(c, launch_shadow_quads(c->d_shadow[level], (int)c->lights[level].shadow_size, c->d_shadowq[level],
+        LAUNCHCHK(c, launch_shadow_pad(c->d_shadow[level], (int)c->lights[level].shadow_size, c->d_shadowp[level],
                                          c->stream));
         HIPCHK(c, hipStreamSynchronize(c->stream));
         return VCT_OK;

@@ -308,7 +308,7 @@ struct ShadowFrag {
     __device__ void finish() {}
 };
 
-__global__ void k_shadow_quads_batch(const DevLight *__restrict__ lights, uint64_t li);
+__global__ void k_shadow_pad_batch(const DevLight *__restrict__ lights, uint64_t li);
 
 hipError_t launch_shadowmaps(const DevScene &sc, const DevLight *hlights, const DevLight *dlights, const int *li,
                              int n, RasterScratch &rs, hipStream_t s) {
@@ -344,51 +344,45 @@ hipError_t launch_shadowmaps(const DevScene &sc, const DevLight *hlights, const 
                                rs.boffs, rs.bchunk, rs.chunk_cap, (int)nslots, fb);
             if ((e = hipGetLastError()) != hipSuccess) return e;
         }
-        // the footprint layout of every map of the walk, one launch
-        int n1max = 0;
+        // the padded copy of every map of the walk, one launch
+        int pmax = 0;
         for (int j = 0; j < nb; ++j) {
             const DevLight &L = hlights[li[j0 + j]];
-            const int n1 = (int)L.shadow_size + 1;
-            if (L.shadowquad && n1 * n1 > n1max) n1max = n1 * n1;
+            if (L.shadowpad) pmax = std::max(pmax, (int)L.shadow_size + 2 * kShadowPad);
         }
-        if (n1max > 0) {
-            hipLaunchKernelGGL(k_shadow_quads_batch, dim3((n1max + 255) / 256, nb), dim3(256), 0, s, dlights, packed);
+        if (pmax > 0) {
+            hipLaunchKernelGGL(k_shadow_pad_batch, dim3(pmax, nb), dim3(256), 0, s, dlights, packed);
             if ((e = hipGetLastError()) != hipSuccess) return e;
         }
     }
     return hipSuccess;
 }
 
-__device__ __forceinline__ void shadow_quad(const float *__restrict__ sm, int N, float4 *q, int idx) {
-    const int n1 = N + 1;
-    const int i = idx % n1 - 1, j = idx / n1 - 1;
-    auto tex = [&](int x, int y) -> float {
-        return (x >= 0 && x < N && y >= 0 && y < N) ? sm[(size_t)y * N + x] : 1.0f;
-    };
-    q[idx] = make_float4(tex(i, j), tex(i + 1, j), tex(i, j + 1), tex(i + 1, j + 1));
+// Row blockIdx.x of a padded copy.
+__device__ __forceinline__ void shadow_pad_row(const float *__restrict__ sm, int N, float *pad) {
+    const int n = N + 2 * kShadowPad, j = (int)blockIdx.x - kShadowPad;
+    if ((int)blockIdx.x >= n) return;
+    for (int x = threadIdx.x; x < n; x += 256) {
+        const int i = x - kShadowPad;
+        pad[(size_t)blockIdx.x * n + x] = (i >= 0 && i < N && j >= 0 && j < N) ? sm[(size_t)j * N + i] : 1.0f;
+    }
 }
 
-__global__ __launch_bounds__(256) void k_shadow_quads(const float *__restrict__ sm, int N, float4 *q) {
-    const int idx = blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx >= (N + 1) * (N + 1)) return;
-    shadow_quad(sm, N, q, idx);
+__global__ __launch_bounds__(256) void k_shadow_pad(const float *__restrict__ sm, int N, float *pad) {
+    shadow_pad_row(sm, N, pad);
 }
 
-// The footprint layouts of a shadow walk's maps: blockIdx.y is the walk's
-// j-th light (its index at bits 5j .. 5j+4 of li); lights without a layout
-// buffer are skipped.
-__global__ __launch_bounds__(256) void k_shadow_quads_batch(const DevLight *__restrict__ lights, uint64_t li) {
+// The padded copies of a shadow walk's maps: blockIdx.y is the walk's j-th
+// light (its index at bits 5j .. 5j+4 of li); lights without a buffer for it
+// are skipped.
+__global__ __launch_bounds__(256) void k_shadow_pad_batch(const DevLight *__restrict__ lights, uint64_t li) {
     const DevLight &L = lights[(li >> (5u * blockIdx.y)) & 31u];
-    const int N = (int)L.shadow_size;
-    const int idx = blockIdx.x * blockDim.x + threadIdx.x;
-    if (!L.shadowquad || idx >= (N + 1) * (N + 1)) return;
-    shadow_quad(L.shadowmap, N, const_cast<float4 *>(L.shadowquad), idx);
+    if (L.shadowpad) shadow_pad_row(L.shadowmap, (int)L.shadow_size, const_cast<float *>(L.shadowpad));
 }
 
-hipError_t launch_shadow_quads(const float *depth, int N, float4 *quads, hipStream_t s) {
-    if (!quads) return hipSuccess;
-    const int n = (N + 1) * (N + 1);
-    hipLaunchKernelGGL(k_shadow_quads, dim3((n + 255) / 256), dim3(256), 0, s, depth, N, quads);
+hipError_t launch_shadow_pad(const float *depth, int N, float *pad, hipStream_t s) {
+    if (!pad) return hipSuccess;
+    hipLaunchKernelGGL(k_shadow_pad, dim3(N + 2 * kShadowPad), dim3(256), 0, s, depth, N, pad);
     return hipGetLastError();
 }
 

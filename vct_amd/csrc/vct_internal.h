@@ -20,6 +20,7 @@ namespace vctk {
 // Light as the kernels see it: the ABI record plus its shadow map pointer.
 constexpr int kMaxLights = 32;  // vct_set_lights
 
+constexpr int kShadowPad = 4;
 struct DevLight {
     float position[3];
     float range;
@@ -31,10 +32,10 @@ struct DevLight {
     float ls[16];
     float ls_inverse[16];
     const float *shadowmap;  // device, shadow_size^2 fp32, row 0 at t = 0
-    // the same map as bilinear footprints: element (i, j), i, j in [-1, N-1],
-    // at (j + 1) * (N + 1) + (i + 1) holds texels (i, j), (i+1, j), (i, j+1),
-    // (i+1, j+1), border texels 1.0 -- one aligned 16-byte load per PCF tap
-    const float4 *shadowquad;
+    // the same map with a border of kShadowPad texels of 1.0 on each side (row
+    // stride shadow_size + 2 kShadowPad): a PCF tap's coordinates need a clamp
+    // only, and the taps' rows are loaded whole
+    const float *shadowpad;
 };
 
 // Radiance pyramid: one device allocation, addressed by 32-bit byte offsets
@@ -222,8 +223,8 @@ inline int shadow_batch(int ntri) {  // slot indices stay below 2^31
 }
 hipError_t launch_shadowmaps(const DevScene &sc, const DevLight *hlights, const DevLight *dlights, const int *li,
                              int n, RasterScratch &rs, hipStream_t s);
-// rebuilds DevLight::shadowquad from the depth map
-hipError_t launch_shadow_quads(const float *depth, int N, float4 *quads, hipStream_t s);
+// rebuilds DevLight::shadowpad from the depth map
+hipError_t launch_shadow_pad(const float *depth, int N, float *pad, hipStream_t s);
 hipError_t launch_gbuffer(const DevScene &sc, const vct_camera &cam, uint64_t *vis, vct_gbuffer_texel *gbuf,
                           RasterScratch &rs, hipStream_t s);
 

@@ -285,7 +285,7 @@ struct VoxFrag {
                         for (int k = 0; k < 3; ++k) lit[h][k] = ((color[k] * L.color[k]) * L.intensity) * ndl;
                     }
                     const bool nz = lit[h][0] != 0.0f || lit[h][1] != 0.0f || lit[h][2] != 0.0f;
-                    fetch[h] = L.shadow_caster && L.shadowquad && __ballot(nz) != 0;  // wave-uniform
+                    fetch[h] = L.shadow_caster && L.shadowpad && __ballot(nz) != 0;  // wave-uniform
                 }
 #pragma unroll
                 for (int h = 0; h < 2; ++h) {
@@ -293,7 +293,7 @@ struct VoxFrag {
                     const DevLight &L = vox_lights[i + h];
                     float w4[4] = {wp[0], wp[1], wp[2], 1.0f}, lsp[4];
                     mat4_vec4(L.ls, w4, lsp);
-                    shadow_taps(lsp, L.shadowquad, (int)L.shadow_size, st[h]);
+                    shadow_taps(lsp, L.shadowpad, (int)L.shadow_size, st[h]);
                 }
 #pragma unroll
                 for (int h = 0; h < 2; ++h) {
@@ -301,7 +301,7 @@ struct VoxFrag {
                     const DevLight &L = vox_lights[i + h];
                     if (!L.enabled) continue;
                     if (fetch[h]) {
-                        const float sf = 1.0f - shadow_count(st[h], (int)L.shadow_size);
+                        const float sf = 1.0f - shadow_count(st[h], L.shadowpad, (int)L.shadow_size);
                         for (int k = 0; k < 3; ++k) lit[h][k] = lit[h][k] * sf;
                     }
                     for (int k = 0; k < 3; ++k) fin[k] = fin[k] + lit[h][k];
