@@ -91,3 +91,36 @@ def test_slot_counts(n):
         assert ctx.stats().total_voxel_fragments == st.total_voxel_fragments
     finally:
         app.close()
+
+
+@pytest.mark.parametrize("n", [70, 2000, 2500, 9000])
+def test_sparse_slots(n):
+    """Chunks of items whose slots lie far apart: all but a few triangles are
+    too small to cover anything, so that a chunk spans from under 64 to
+    thousands of slots; items of both passes, samples and statistics."""
+    app = make_app(1, dim=64)
+    try:
+        ctx, fs = app.ctx, app.frame_state(0)
+        eye = np.eye(4, dtype=np.float32)[None]
+        m = _soup(app.mesh()["pos"], n, n)
+        c = m["pos"].mean(1, keepdims=True)
+        scale = np.full((n, 1, 1), 1e-6, np.float32)
+        scale[:: max(1, n // 12)] = 0.05  # a dozen of a few pixels each
+        scale[n // 2:: max(1, n // 3)] = 1.0
+        m["pos"] = (c + (m["pos"] - c) * scale).astype(np.float32)
+        ctx.set_scene(m["pos"], m["nrm"], m["tan"], m["albedo"], m["obj"], 1)
+        ctx.set_transforms(eye)
+        sc = ob.SceneArrays(m, eye)
+        L = abi.Light.from_buffer_copy(next(L for L in fs["lights"] if L.shadow_caster))
+        L.shadow_size = 256
+        ctx.set_lights([L])
+        ctx.shadowmaps()
+        ref = ob.shadowmap(sc, L)
+        assert np.array_equal(ctx.shadow(0).view(np.uint32), ref.view(np.uint32))
+        ctx.voxelize(fs["vox"])
+        alb, nrm, st = ob.voxelize(sc, [L], [ref], fs["vox"], 64)
+        assert (alb != 0).any()
+        assert np.array_equal(ctx.albedo(), alb) and np.array_equal(ctx.normal(), nrm)
+        assert ctx.stats().total_voxel_fragments == st.total_voxel_fragments
+    finally:
+        app.close()

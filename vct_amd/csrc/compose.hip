@@ -47,8 +47,9 @@ __device__ __forceinline__ void cook_torrance(const float lambert[3], const floa
     }
 }
 
-__device__ __forceinline__ float smoothstep_gl(float e0, float e1, float x) {
-    const float t = clampf((x - e0) / (e1 - e0), 0.0f, 1.0f);
+// smoothstep(e0, e1, x), given RN64(1 / (e1 - e0))
+__device__ __forceinline__ float smoothstep_gl(float e0, double rcp, float x) {
+    const float t = clampf(quot_f32(x - e0, rcp), 0.0f, 1.0f);
     return (t * t) * (3.0f - 2.0f * t);
 }
 
@@ -95,11 +96,10 @@ __global__ __launch_bounds__(256) void k_compose(ComposeArgs a) {
             const float d[3] = {Lt.position[0] - P[0], Lt.position[1] - P[1], Lt.position[2] - P[2]};
             const float dist = sqrtf(dot3(d, d));
             if (dist > Lt.range) continue;
-            att = 1.0f - smoothstep_gl(0.75f * Lt.range, Lt.range, dist);
+            att = 1.0f - smoothstep_gl(Lt.fade0, Lt.rcp_fade, dist);
             nrm3(d, Ld);
         } else {  // directional (phong.frag:290-302)
-            const float nd[3] = {-Lt.direction[0], -Lt.direction[1], -Lt.direction[2]};
-            nrm3(nd, Ld);
+            for (int c = 0; c < 3; ++c) Ld[c] = Lt.to_light[c];
         }
         const float vl[3] = {V[0] + Ld[0], V[1] + Ld[1], V[2] + Ld[2]};
         float H[3];

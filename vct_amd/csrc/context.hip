@@ -709,6 +709,18 @@ int vct_set_transforms(vct_ctx *c, const float *model, int n) {
     return VCT_OK;
 }
 
+// What the shaders compute of a light alone, in their operations: every one is
+// IEEE float or double arithmetic, so the bits are those a fragment would get.
+static void light_constants(DevLight &d) {
+#pragma clang fp contract(off)
+    const float v[3] = {-d.direction[0], -d.direction[1], -d.direction[2]};
+    const float l = std::sqrt((v[0] * v[0] + v[1] * v[1]) + v[2] * v[2]);
+    const double r = 1.0 / (double)l;
+    for (int k = 0; k < 3; ++k) d.to_light[k] = (float)((double)v[k] * r);
+    d.fade0 = 0.75f * d.range;
+    d.rcp_fade = 1.0 / (double)(d.range - d.fade0);
+}
+
 int vct_set_lights(vct_ctx *c, const vct_light *lights, int n) {
     if (!c || (n > 0 && !lights)) return fail(c, VCT_ERR_INVALID, "vct_set_lights: NULL argument");
     if (n < 0 || n > kMaxLights) return fail(c, VCT_ERR_INVALID, "vct_set_lights: %d lights (max %d)", n, kMaxLights);
@@ -761,6 +773,7 @@ int vct_set_lights(vct_ctx *c, const vct_light *lights, int n) {
         memcpy(d.ls_inverse, L.ls_inverse, 64);
         d.shadowmap = maps[i];
         d.shadowpad = pads[i];
+        light_constants(d);
     }
     dfree(c->d_lights);
     if (n) {

@@ -82,7 +82,7 @@ __global__ __launch_bounds__(256) void k_inject_scatter(InjectBatch B, int dim, 
     float ndc4[4] = {tcx * 2.0f - 1.0f, tcy * 2.0f - 1.0f, d * 2.0f - 1.0f, 1.0f}, w[4];
     mat4_vec4(L.ls_inverse, ndc4, w);
     if (L.perspective) {
-        const double rw = 1.0 / (double)w[3];
+        const double rw = rcp_f64(w[3]);
         w[0] = quot_f32(w[0], rw);
         w[1] = quot_f32(w[1], rw);
         w[2] = quot_f32(w[2], rw);

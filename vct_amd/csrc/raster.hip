@@ -149,11 +149,6 @@ __global__ __launch_bounds__(256) void k_shadow_setup(DevScene sc, const DevLigh
 
 constexpr int kBlockRun = 64;
 
-__device__ __forceinline__ uint64_t readlane_u64(uint64_t v, int lane) {
-    return ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(v >> 32), lane) << 32) |
-           (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)v, lane);
-}
-
 template <class F>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void k_raster_blocks(
     const int4 *__restrict__ recs, const uint64_t *__restrict__ offs, const uint32_t *__restrict__ chunk,
@@ -202,7 +197,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void k
             const uint32_t local = (uint32_t)(k - t0);  // the run may enter a triangle mid-way
             uint32_t bxi = __builtin_amdgcn_readfirstlane(local % nbx);
             const int bx0 = (e.x0 >> 3) * 8, by = ((e.y0 >> 3) + (int)(local / nbx)) * 8;
-            const double rcp = 1.0 / (double)e.area;  // RN64(1 / area)
+            const double rcp = rcp_f64(e.area);
             double E[3], row[3], As[3], Bs[3], lim[3];
 #pragma unroll
             for (int i = 0; i < 3; ++i) {
@@ -546,7 +541,7 @@ __global__ __launch_bounds__(256) void k_gbuf_resolve(DevScene sc, CamMats cm, c
     b[1] = ax[2] * ay[0] - ay[2] * ax[0];
     b[2] = ax[0] * ay[1] - ay[0] * ax[1];
     const float sum = (b[0] + b[1]) + b[2];
-    const double rsum = 1.0 / (double)sum;  // the three IEEE quotients b[v] / sum (quot_f32)
+    const double rsum = rcp_f64(sum);  // the three IEEE quotients b[v] / sum (quot_f32)
     for (int v = 0; v < 3; ++v) b[v] = quot_f32(b[v], rsum);
     const float *Nm = sc.nmat + (size_t)sc.obj[t] * 9;
     float Tw[3];

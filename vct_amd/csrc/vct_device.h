@@ -21,8 +21,8 @@ __device__ __forceinline__ float dot3(const float a[3], const float b[3]) {
 }
 // a / b correctly rounded to float (the IEEE division a / b), for finite
 // floats a and b != 0 whose quotient is a normal float or zero, given rcp =
-// RN64(1 / b).  q = RN64(a * rcp) is within (1 + 2^-53)^2 - 1 < 2^-52 of a / b,
-// relatively.  A rounding boundary of float is a midpoint m = M 2^k, M odd
+// RN64(1 / b) or rcp_f64(b), within 2^-52 of 1 / b.  q = RN64(a * rcp) is within
+// 2^-51 of a / b, relatively.  A rounding boundary of float is a midpoint m = M 2^k, M odd
 // with 25 bits; with |a| = A 2^i, |b| = B 2^j (A, B < 2^24), |a| - m |b| is a
 // nonzero multiple of 2^min(i, k + j) (it is never zero: A would need the odd
 // factor M), so ||a / b| - m| >= 2^-50 |a / b|.  q therefore rounds to float
@@ -30,11 +30,23 @@ __device__ __forceinline__ float dot3(const float a[3], const float b[3]) {
 // symmetric in sign): RN32(q) = RN32(a / b).
 __device__ __forceinline__ float quot_f32(float a, double rcp) { return (float)((double)a * rcp); }
 
+// 1 / b for quot_f32 in half the operations of the FP64 division: the hardware's
+// estimate and two Newton steps, each of which squares its relative error (2^-14
+// would do) up to the rounding of its last operation, so that the result is within
+// 2^-52; div_fixup gives 0, infinity and NaN what the division gives them.
+__device__ __forceinline__ double rcp_f64(float b) {
+    const double d = (double)b;
+    double r = __builtin_amdgcn_rcp(d);
+    r = fma(r, fma(-d, r, 1.0), r);
+    r = fma(r, fma(-d, r, 1.0), r);
+    return __builtin_amdgcn_div_fixup(r, d, 1.0);
+}
+
 // v / length(v), each component the IEEE quotient v[k] / l (quot_f32 with one
 // FP64 reciprocal instead of three float divisions)
 __device__ __forceinline__ void nrm3(const float v[3], float o[3]) {
     const float l = __builtin_sqrtf(dot3(v, v));
-    const double r = 1.0 / (double)l;
+    const double r = rcp_f64(l);
     o[0] = quot_f32(v[0], r);
     o[1] = quot_f32(v[1], r);
     o[2] = quot_f32(v[2], r);
@@ -289,7 +301,7 @@ __device__ __forceinline__ void shadow_taps(const float lsp[4], const float *pad
     if (__ballot(lsp[3] != 1.0f) == 0) {  // orthographic light space: w = 1, and x / 1 is x
         for (int k = 0; k < 3; ++k) sh[k] = (lsp[k] + 1.0f) * 0.5f;
     } else {
-        const double rw = 1.0 / (double)lsp[3];  // the three IEEE quotients by w (quot_f32)
+        const double rw = rcp_f64(lsp[3]);  // the three IEEE quotients by w (quot_f32)
         for (int k = 0; k < 3; ++k) sh[k] = (quot_f32(lsp[k], rw) + 1.0f) * 0.5f;
     }
     st.s = sh[0];
@@ -373,6 +385,10 @@ __device__ __forceinline__ T seen(const T *p) {
 
 // ---- wave helpers ----------------------------------------------------------
 __device__ __forceinline__ int lane_id() { return __lane_id(); }
+__device__ __forceinline__ uint64_t readlane_u64(uint64_t v, int lane) {
+    return ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(v >> 32), lane) << 32) |
+           (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)v, lane);
+}
 
 // Reduces (sum a, max b, sum c, sum d) over a 256-thread workgroup and writes
 // them to partials[blockIdx.x * 4 ..].  Every thread of the block must call it.

@@ -36,6 +36,9 @@ struct DevLight {
     // stride shadow_size + 2 kShadowPad): a PCF tap's coordinates need a clamp
     // only, and the taps' rows are loaded whole
     const float *shadowpad;
+    float to_light[3];  // directional: -direction, normalized
+    float fade0;        // point: the attenuation's start, 0.75 range ...
+    double rcp_fade;    // ... and RN64(1 / (range - fade0))
 };
 
 // Radiance pyramid: one device allocation, addressed by 32-bit byte offsets

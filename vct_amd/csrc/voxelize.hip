@@ -102,6 +102,24 @@ __device__ __forceinline__ bool vox_cover(const float4 *attr, int msaa, int slot
         // ndc z of the three vertices: f[2], f[5], f[8]
         const float nz0 = a[0].z, nz1 = a[1].y, nz2 = a[2].x;
         bool cov = false;
+        if (e.small && msaa && !zclip) {
+            // the four samples without a branch between them: the edges at the
+            // pixel's corner, the samples (3, 1) (7, 3) (1, 5) (5, 7) in 1/8 px
+            const int dx = (px - e.x0) << 8, dy = (py - e.y0) << 8;
+            int in[4];
+#pragma unroll
+            for (int i = 0; i < 3; ++i) {
+                const uint32_t c = (uint32_t)(e.E0[i] + __mul24(e.A[i], dx) + __mul24(e.B[i], dy) + e.bias[i]);
+                const uint32_t a = (uint32_t)e.A[i] << 5, b = (uint32_t)e.B[i] << 5;
+                const uint32_t v[4] = {c + (a * 2 + a) + b, c + (a * 8 - a) + (b * 2 + b), c + a + (b * 4 + b),
+                                       c + (a * 4 + a) + (b * 8 - b)};
+#pragma unroll
+                for (int k = 0; k < 4; ++k) in[k] = i == 0 ? (int)v[k] : in[k] | (int)v[k];  // negative: outside an edge
+            }
+            if ((in[0] & in[1] & in[2] & in[3]) < 0) return false;  // no sample inside all three
+            edge_bary(e, px, py, 128, 128, l);
+            return true;
+        }
         const int ns = msaa ? 4 : 1;
         for (int k = 0; k < ns && !cov; ++k) {
             const int ox = msaa ? msaa_x(k) : 128, oy = msaa ? msaa_y(k) : 128;
@@ -164,7 +182,7 @@ __device__ __forceinline__ void rgba8_avg(uint32_t *p, float r, float g, float b
         c2 = c2 * c3;
         float s0 = c0 + v0, s1 = c1 + v1, s2 = c2 + v2;
         const float s3 = c3 + v3;
-        const double r3 = 1.0 / (double)s3;  // the three IEEE quotients by s3 (quot_f32)
+        const double r3 = rcp_f64(s3);  // the three IEEE quotients by s3 (quot_f32)
         s0 = quot_f32(s0, r3);
         s1 = quot_f32(s1, r3);
         s2 = quot_f32(s2, r3);
@@ -273,15 +291,12 @@ struct VoxFrag {
                         const float ndl = __builtin_fmaxf(0.0f, dot3(nn, dn));
                         for (int k = 0; k < 3; ++k) lit[h][k] = ((color[k] * L.intensity) * L.color[k]) * ndl;
                         const float dist = __builtin_sqrtf(dot3(d, d));
-                        const float e0 = 0.75f * L.range, e1 = L.range;
-                        const float tt = clampf((dist - e0) / (e1 - e0), 0.0f, 1.0f);
+                        const float tt = clampf(quot_f32(dist - L.fade0, L.rcp_fade), 0.0f, 1.0f);
                         const float ss = (tt * tt) * (3.0f - 2.0f * tt);
                         const float att = 1.0f - ss;
                         for (int k = 0; k < 3; ++k) lit[h][k] = lit[h][k] * att;
                     } else {
-                        float nd[3] = {-L.direction[0], -L.direction[1], -L.direction[2]}, ndn[3];
-                        nrm3(nd, ndn);
-                        const float ndl = __builtin_fmaxf(0.0f, dot3(nn, ndn));
+                        const float ndl = __builtin_fmaxf(0.0f, dot3(nn, L.to_light));
                         for (int k = 0; k < 3; ++k) lit[h][k] = ((color[k] * L.color[k]) * L.intensity) * ndl;
                     }
                     const bool nz = lit[h][0] != 0.0f || lit[h][1] != 0.0f || lit[h][2] != 0.0f;
@@ -635,25 +650,20 @@ __global__ __launch_bounds__(256) void k_tess_points(DevScene sc, TessArgs ta, c
                                                      const float4 *__restrict__ attr, const uint64_t *__restrict__ offs,
                                                      const uint32_t *__restrict__ chunk, size_t chunk_cap, int accum,
                                                      uint32_t *albedo, uint32_t *normal) {
+    __shared__ uint32_t marks[4][64];
     const int nslots = sc.ntri;
     const uint64_t total = offs[nslots];
     const uint64_t nchunks = (total + 63) >> 6;
-    for (uint64_t k = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; k < total;
-         k += (uint64_t)gridDim.x * blockDim.x) {
-        const uint64_t c = k >> 6;
-        int lo = c < chunk_cap ? (int)chunk[c] : 0;
-        int hi = (c + 1 < nchunks && c + 1 < chunk_cap) ? (int)chunk[c + 1] : nslots - 1;
-        while (lo < hi) {
-            const int mid = (lo + hi + 1) >> 1;
-            if (offs[mid] <= k) lo = mid;
-            else hi = mid - 1;
-        }
-        const int t = lo;
-        const int j = (int)(k - offs[t]);
+    const int lane = threadIdx.x & 63;
+    const uint64_t wave = ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
+    for (uint64_t c = wave; c < nchunks; c += ((uint64_t)gridDim.x * blockDim.x) >> 6) {
+        int t;
+        const uint32_t j = chunk_item(offs, chunk, chunk_cap, nslots, nchunks, c, lane, marks[threadIdx.x >> 6], t);
+        if ((c << 6) + (uint64_t)lane >= total) continue;
         const int4 r = rec[(size_t)t * 4];
         const int lv[4] = {r.x, r.y, r.z, r.w};
         float w[3];
-        tess_point(lv, j, w);
+        tess_point(lv, (int)j, w);
         const float4 *a = attr + (size_t)t * 8;
         const float4 a0 = a[0], a1 = a[1], a2 = a[2], a3 = a[3], a4 = a[4];
         const float P[3][3] = {{a0.x, a0.y, a0.z}, {a0.w, a1.x, a1.y}, {a1.z, a1.w, a2.x}};
