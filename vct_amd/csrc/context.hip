@@ -1419,7 +1419,7 @@ int vct_learned_prepare(vct_ctx *c) {
     if (rc) return rc;
     if (!c->d_points) return fail(c, VCT_ERR_STATE, "vct_learned_prepare: no points");
     const Extent e = ctx_extent(c);
-    LAUNCHCHK(c, launch_label64(c->pyr, c->pyr_nonneg ? 1 : 0, c->d_points, c->npoints, e, c->d_labels, c->stream));
+    LAUNCHCHK(c, launch_label64(c->pyr, c->d_points, c->npoints, e, c->d_labels, c->stream));
     LAUNCHCHK(c, launch_features(c->pyr, c->d_points, c->npoints, e, c->d_X, c->stream));
     // output scale: the mean label magnitude, so the network fits O(1) targets
     std::vector<float> lab((size_t)c->npoints * 4);
@@ -1581,7 +1581,7 @@ int vct_reference_gather(vct_ctx *c) {
     if (rc) return rc;
     if (!c->have_gbuf) return fail(c, VCT_ERR_STATE, "vct_reference_gather: no G-buffer");
     if (!c->d_reference) HIPCHK(c, dalloc(&c->d_reference, (size_t)c->gw * c->gh * 16));
-    LAUNCHCHK(c, launch_label64(c->pyr, c->pyr_nonneg ? 1 : 0, c->d_gbuf, c->gw * c->gh, ctx_extent(c), c->d_reference, c->stream));
+    LAUNCHCHK(c, launch_label64(c->pyr, c->d_gbuf, c->gw * c->gh, ctx_extent(c), c->d_reference, c->stream));
     return VCT_OK;
 }
 

@@ -25,8 +25,7 @@ struct MlpBuffers {
     float out_scale = 1.0f;
 };
 
-// nested: TraceLaunch::nested
-hipError_t launch_label64(const PyrDesc &pyr, int nested, const vct_gbuffer_texel *pts, int npts, Extent ext, float4 *out,
+hipError_t launch_label64(const PyrDesc &pyr, const vct_gbuffer_texel *pts, int npts, Extent ext, float4 *out,
                           hipStream_t s);
 hipError_t launch_features(const PyrDesc &pyr, const vct_gbuffer_texel *pts, int npts, Extent ext, uint16_t *X,
                            hipStream_t s);

@@ -52,6 +52,68 @@ struct PyrView {
     LevelInfo l2;
 };
 
+// GL LINEAR inside face 0 of one level (border 0), FP32 weights and sums.
+// p in [0,1]^3 texture coordinates; s = the level's edge.
+__device__ __forceinline__ float4 level_linear(const char *pyr, const LevelInfo &L, const float p[3]) {
+    const int s = L.size;
+    int i0[3];
+    float f[3];
+    for (int k = 0; k < 3; ++k) {
+        const float u = p[k] * (float)s - 0.5f;
+        const float fl = __builtin_floorf(u);
+        i0[k] = (int)fl;
+        f[k] = u - fl;
+    }
+    float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (L.fmt == 0) {  // fp16 pairs: one load per (y, z) corner pair
+        const bool xin = i0[0] >= 0 && i0[0] < s;  // i0 = s - 1 reads the zero border half
+        const bool xneg = i0[0] == -1;
+        if (!xin && !xneg) return acc;
+        const int cx = xneg ? 0 : i0[0];
+        const float wlo = xneg ? f[0] : 1.0f - f[0], whi = xneg ? 0.0f : f[0];
+        for (int c = 0; c < 4; ++c) {
+            const int dy = c & 1, dz = c >> 1;
+            const int y = i0[1] + dy, z = i0[2] + dz;
+            if ((unsigned)y >= (unsigned)s || (unsigned)z >= (unsigned)s) continue;
+            const float wyz = (dy ? f[1] : 1.0f - f[1]) * (dz ? f[2] : 1.0f - f[2]);
+            const uint4 v = *(const uint4 *)(pyr + L.base + (size_t)elem_index(L, cx, y, z, 0) * 16);
+            const float4 lo = unpack_h4(v.x, v.y), hi = unpack_h4(v.z, v.w);
+            const float a = wlo * wyz, b = whi * wyz;
+            acc.x += a * lo.x + b * hi.x;
+            acc.y += a * lo.y + b * hi.y;
+            acc.z += a * lo.z + b * hi.z;
+            acc.w += a * lo.w + b * hi.w;
+        }
+        return acc;
+    }
+    for (int c = 0; c < 8; ++c) {
+        const int dx = c & 1, dy = (c >> 1) & 1, dz = c >> 2;
+        const int x = i0[0] + dx, y = i0[1] + dy, z = i0[2] + dz;
+        if ((unsigned)x >= (unsigned)s || (unsigned)y >= (unsigned)s || (unsigned)z >= (unsigned)s) continue;
+        const float w = ((dx ? f[0] : 1.0f - f[0]) * (dy ? f[1] : 1.0f - f[1])) * (dz ? f[2] : 1.0f - f[2]);
+        // fp32 elements, or the decoded copy of an fp8 level
+        const float4 t = *(const float4 *)(pyr + L.stage + (size_t)elem_index(L, x, y, z, 0) * 16);
+        acc.x += w * t.x;
+        acc.y += w * t.y;
+        acc.z += w * t.z;
+        acc.w += w * t.w;
+    }
+    return acc;
+}
+
+// textureLod with LINEAR_MIPMAP_LINEAR on an isotropic pyramid (border 0).
+__device__ __forceinline__ float4 sample_iso(const PyrView &v, const float p[3], float lam) {
+    const int q = v.nlevels - 1;
+    if (!(lam < (float)q)) return level_linear(v.pyr, v.lv[q], p);
+    if (lam < 0.0f) lam = 0.0f;
+    int d1 = (int)floorf(lam);
+    d1 = d1 > q - 1 ? q - 1 : d1;
+    const float fr = lam - (float)d1;
+    const float4 a = level_linear(v.pyr, v.lv[d1], p), b = level_linear(v.pyr, v.lv[d1 + 1], p);
+    return make_float4((1.0f - fr) * a.x + fr * b.x, (1.0f - fr) * a.y + fr * b.y, (1.0f - fr) * a.z + fr * b.z,
+                       (1.0f - fr) * a.w + fr * b.w);
+}
+
 // ---------------------------------------------------------------- labels
 // 64 directions: Fibonacci set uniform in cos(theta) around local +y;
 // weights y_i / 32 (sum 1).  Same definition as the oracle's or_label.c.
@@ -66,38 +128,10 @@ __device__ __forceinline__ void label_dir(int i, double d[3], double *w) {
     *w = y / 32.0;
 }
 
-// The march's schedule: h_i, and the level class and fraction of
-// log2(max(1, 2 h_i tan)) + 0.5, depend on the step alone.  From h = 1 a step
-// grows h by 1 + tan(10 deg) / 2, and a sample further than sqrt(3) dim voxels
-// from a start inside the grid is outside it: at most 82 steps for dim 512, so
-// the reference's 256-step limit is never reached and `n` entries cover every
-// cone (h_{n-1} > sqrt(3) dim).
-constexpr int kLabelSteps = 96;
-struct LabelSchedule {
-    int n;
-    double h[kLabelSteps];
-    int cls[kLabelSteps];
-    float fr[kLabelSteps];
-};
-
-// One wavefront per point, one cone per lane.  The lanes' cells differ, so a
-// sample is per-lane loads: what bounds it is the texture-address unit and the
-// FP64 accumulation.  The schedule comes from the kernel arguments (FP64
-// log2 per step and lane before), levels are sampled by the tracer's sampler
-// (scalar loads where the lanes share a cell, the finer level skipped under an
-// empty coarser one), a step that is empty in every lane skips the FP64 square
-// root and sums, and a wavefront takes several points, so that the cone
-// directions (FP64 sine and cosine) are set up once.  32,768 points, 64^3:
-// 1276 us before, 805 us now.
-template <int MODE>
-__global__ __launch_bounds__(64) void k_label64(const vct_gbuffer_texel *__restrict__ pts, int npts, PyrArgs pa,
-                                                LabelSchedule sc, Extent ext, float4 *out) {
-    const int dim = pa.dim;
+__global__ __launch_bounds__(64) void k_label64(const vct_gbuffer_texel *__restrict__ pts, int npts, PyrView pv,
+                                                Extent ext, float4 *out) {
+    const int dim = pv.dim;
     const int lane = threadIdx.x;
-    const __amdgpu_buffer_rsrc_t rs = pyr_rsrc(pa);
-    double dl[3], w;
-    label_dir(lane, dl, &w);
-    const ConeFaces cf = {{0u, 0u, 0u}, {0u, 0u, 0u}, {0.f, 0.f, 0.f}, 0u, true};
     for (int pi = blockIdx.x; pi < npts; pi += gridDim.x) {
         const float4 *g = (const float4 *)&pts[pi];
         const float4 g0 = g[0], g1 = g[1], g2 = g[2], g3 = g[3];
@@ -114,28 +148,31 @@ __global__ __launch_bounds__(64) void k_label64(const vct_gbuffer_texel *__restr
         N[2] = g1.z / n2;
         for (int k = 0; k < 3; ++k)
             pos[k] = ((double)gp[k] - ext.center[k] - ext.vmin[k]) / ((double)ext.vmax[k] - ext.vmin[k]);
+        double dl[3], w;
+        label_dir(lane, dl, &w);
         double d[3] = {g2.x * dl[0] + g3.x * dl[1] + g1.x * dl[2], g2.y * dl[0] + g3.y * dl[1] + g1.y * dl[2],
                        g2.z * dl[0] + g3.z * dl[1] + g1.z * dl[2]};
         const double dn = sqrt(d[0] * d[0] + d[1] * d[1] + d[2] * d[2]);
         for (int k = 0; k < 3; ++k) d[k] /= dn;
+        const double tan_half = 0.17632698070846498;  // tan(10 degrees)
         const double scale = 1.0 / dim;
         double start[3];
         for (int k = 0; k < 3; ++k) start[k] = pos[k] + N[k] * scale;
-        double c0 = 0, c1 = 0, c2 = 0, a = 0;
-        for (int i = 0; i < sc.n && a < 0.999; ++i) {
-            const double h = sc.h[i];
+        double c0 = 0, c1 = 0, c2 = 0, a = 0, h = 1.0;
+        for (int i = 0; i < 256 && a < 0.999; ++i) {
+            const double r = h * tan_half;
+            const double lod = log2(fmax(1.0, 2.0 * r)) + 0.5;
             float sp[3];
             bool outside = false;
+            double spd[3];
             for (int k = 0; k < 3; ++k) {
-                const double spd = start[k] + h * d[k] * scale;
-                if (spd < 0.0 || spd > 1.0) outside = true;
-                sp[k] = (float)spd;
+                spd[k] = start[k] + h * d[k] * scale;
+                if (spd[k] < 0.0 || spd[k] > 1.0) outside = true;
+                sp[k] = (float)spd[k];
             }
             if (outside) break;
             // trilinear sampling in FP32; transmittance and radiance accumulate in FP64
-            const float4 s = sample_class<MODE>(pa, rs, sc.cls[i], sc.fr[i], sp, cf);
-            // nothing in any lane's sample: the sums below would all add 0
-            if (__ballot(s.x != 0.f || s.y != 0.f || s.z != 0.f || s.w != 0.f) == 0) continue;
+            const float4 s = sample_iso(pv, sp, (float)lod);
             double sa = s.w < 0.f ? 0.0 : (s.w > 1.f ? 1.0 : (double)s.w);
             const double ah = 1.0 - sqrt(1.0 - sa);
             const double tr = 1.0 - a;
@@ -143,6 +180,7 @@ __global__ __launch_bounds__(64) void k_label64(const vct_gbuffer_texel *__restr
             c1 += 0.5 * s.y * tr;
             c2 += 0.5 * s.z * tr;
             a += tr * ah;
+            h += 0.5 * r;
         }
         double v[4] = {w * c0, w * c1, w * c2, w * a};
         for (int off = 32; off > 0; off >>= 1)
@@ -1133,40 +1171,10 @@ static PyrView pyr_view(const PyrDesc &pyr) {
     return v;
 }
 
-static LabelSchedule label_schedule(int dim, int nlevels) {
-    LabelSchedule sc;
-    const double tan_half = 0.17632698070846498;  // tan(10 degrees)
-    const int q = nlevels - 1;
-    double h = 1.0;
-    sc.n = 0;
-    while (sc.n < kLabelSteps) {
-        const int i = sc.n++;
-        const double r = h * tan_half;
-        const float lam = (float)(log2(fmax(1.0, 2.0 * r)) + 0.5);
-        sc.h[i] = h;
-        sc.cls[i] = lam < (float)q ? (int)floorf(lam) : q;
-        sc.fr[i] = lam < (float)q ? lam - floorf(lam) : 0.0f;
-        if (h > 1.7320508075688774 * dim) break;
-        h += 0.5 * r;
-    }
-    return sc;
-}
-
-// Wavefronts of a label launch: enough to fill the device several times over,
-// few enough that one takes several points.
-constexpr int kLabelBlocks = 16384;
-
-hipError_t launch_label64(const PyrDesc &pyr, int nested, const vct_gbuffer_texel *pts, int npts, Extent ext, float4 *out,
+hipError_t launch_label64(const PyrDesc &pyr, const vct_gbuffer_texel *pts, int npts, Extent ext, float4 *out,
                           hipStream_t s) {
-    const int blocks = npts < kLabelBlocks ? (npts > 0 ? npts : 1) : kLabelBlocks;
-    const LabelSchedule sc = label_schedule(pyr.dim, pyr.nlevels);
-    const PyrArgs pa = pyr_args(pyr, nested);
-    if (pyr.storage == VCT_STORE_FP32)
-        hipLaunchKernelGGL(k_label64<1>, dim3(blocks), dim3(64), 0, s, pts, npts, pa, sc, ext, out);
-    else if (pyr.storage == VCT_STORE_FP8)
-        hipLaunchKernelGGL(k_label64<2>, dim3(blocks), dim3(64), 0, s, pts, npts, pa, sc, ext, out);
-    else
-        hipLaunchKernelGGL(k_label64<0>, dim3(blocks), dim3(64), 0, s, pts, npts, pa, sc, ext, out);
+    const int blocks = npts < 65536 ? (npts > 0 ? npts : 1) : 65536;
+    hipLaunchKernelGGL(k_label64, dim3(blocks), dim3(64), 0, s, pts, npts, pyr_view(pyr), ext, out);
     return hipGetLastError();
 }
 
