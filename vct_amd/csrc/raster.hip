@@ -52,6 +52,26 @@ __device__ __forceinline__ uint64_t bbox_blocks(const int4 r[4], uint64_t cnt) {
     return nbx * nby;
 }
 
+// A record for the block walk, whose FP64 sums start from the edge values C at the
+// origin, every sum exact.  |A|, |B| <= 2^28 and a pixel centre is below 2^22 in
+// 1/256 px, an odd multiple of 128: the terms in A and B are multiples of 128 and
+// together at most 2^51.  With C below 2^52 every sum is an integer below 2^53.  From
+// there on (C is at most 2^55) the edge passes far from the image: no sum changes its
+// sign, and the values lie between 2^51 and 2^56, where floats and the midpoints
+// between them are multiples of 2^27.  So all values from one multiple of 128 to the
+// next, ends excluded, round to the same float, and C's remainder mod 128 may be 64
+// wherever it is not 0: multiples of 64 below 2^56 are exact again.
+__device__ __forceinline__ void walk_record(int4 r[4]) {
+    if (((uint32_t)r[1].w >> 19) & 1u) return;  // small: 32-bit values
+    int *const w[3][2] = {{&r[2].x, &r[2].y}, {&r[2].z, &r[2].w}, {&r[3].x, &r[3].y}};
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+        const int64_t c = (int64_t)(((uint64_t)(uint32_t)*w[i][1] << 32) | (uint32_t)*w[i][0]);
+        const bool far = (uint64_t)(c + ((int64_t)1 << 52)) >= ((uint64_t)1 << 53);
+        if (far) *w[i][0] = (*w[i][0] & ~127) | ((*w[i][0] & 127) ? 64 : 0);
+    }
+}
+
 // Words of `w` to v, by `threads` threads of which this is the t-th: 16 bytes
 // at a time (w is the start of an allocation).
 __device__ __forceinline__ void fill_words(uint32_t *w, uint32_t v, size_t n, size_t t, size_t threads) {
@@ -103,6 +123,7 @@ __global__ __launch_bounds__(256) void k_shadow_setup(DevScene sc, const DevLigh
         // (Application.cpp:737,942,979); the record's user field is the light
         cnt = tri_setup(win, N, N, 1, l, r);
         if (cnt) {
+            if (cnt > kBlockPixels) walk_record(r);
             for (int i = 0; i < 4; ++i) rec[slot * 4 + i] = r[i];
             attr[slot] = make_float4(zw[0], zw[1], zw[2], 0.0f);
         }
@@ -124,11 +145,10 @@ __global__ __launch_bounds__(256) void k_shadow_setup(DevScene sc, const DevLigh
 // the lanes hold, read where a run begins or passes their end.  (A table of every
 // block's slot, filled by a launch of its own, took 10 to 23 us and left the walk
 // no faster: 534 us with it, 507 without.)  Each lane keeps its three edge values
-// in FP64 and steps them from block to block: every one is an integer below 2^53
-// (|A|, |B| <= 2^28, a coordinate in 1/256 px below 2^22), so every sum is exact,
-// the values are those of edge_value in both of its forms, and the barycentrics are
-// quot_f32(E, area) with the triangle's reciprocal: every fragment and its
-// barycentrics are those the pixel walk produces.  F provides Tri (a triangle's
+// in FP64 and steps them from block to block, every sum exact (walk_record), so the
+// values round to float as those of edge_value do in both of its forms, and the
+// barycentrics are quot_f32(E, area) with the triangle's reciprocal: every fragment
+// and its barycentrics are those the pixel walk produces.  F provides Tri (a triangle's
 // wave-uniform data, the image size W x H among it), enter(slot, edges) that
 // gives it, and three stages of a fragment, between which a Pending goes:
 // fetch(tri, px, py, in), depth(tri, l, pending) and store(pending), which runs
@@ -438,6 +458,7 @@ __global__ __launch_bounds__(256) void k_gbuf_setup(DevScene sc, CamMats cm, int
                 int4 r[4];
                 cnt = tri_setup(win, cm.W, cm.H, cm.cull, t, r);
                 if (cnt) {
+                    if (cnt > kBlockPixels) walk_record(r);
                     for (int i = 0; i < 4; ++i) rec[slot * 4 + i] = r[i];
                     attr[slot] = make_float4(zw[0], zw[1], zw[2], 0.0f);
                 }
