@@ -55,7 +55,7 @@ def test_whole_tiles(storage, aniso, warp):
         p = parts[1]
         for a, r in zip(whole, ob.trace(np.ascontiguousarray(gbuf[p]), levels, tp, aniso_faces=faces)):
             assert rel_err(a[p].reshape(-1, 4), r) < 1e-3, rel_err(a[p].reshape(-1, 4), r)
-        # without the specular cone the grid holds the tiles once
+        # without the specular cone
         one = abi.TraceParams.from_buffer_copy(tr)
         one.enable_reflections = 0
         assert np.array_equal(_trace(ctx, cam, one, gbuf)[0].view(np.uint32), whole[0].view(np.uint32))
@@ -67,5 +67,30 @@ def test_whole_tiles(storage, aniso, warp):
         keep[:, ::3] = keep[::5, 1::5] = False
         for a, b in zip(whole, _trace(ctx, cam, tr, bad)):
             assert np.array_equal(a[keep].view(np.uint32), b[keep].view(np.uint32))
+    finally:
+        app.close()
+
+
+@pytest.mark.parametrize("warp", [0, 1])
+@pytest.mark.parametrize("aniso", [0, 1])
+def test_without_specular_cone(aniso, warp):
+    """The sizes at which a launch of the diffuse cones alone changes its form:
+    4096 | 4160 tiles (six directions), 8192 | 8320 (isotropic), 9216 | 9288 (six
+    directions, warped)."""
+    w, h = 1320, 680
+    app = make_app(1, dim=32, anisotropic=aniso, width=w, height=h, shadow_size=128, warp_texture=warp, reflections=0)
+    try:
+        ctx, fs = app.ctx, app.frame_state(0)
+        app.render(0)
+        cam, tr = fs["cam"], fs["trace"]
+        assert not tr.enable_reflections
+        gbuf = ctx.download(abi.VCT_BUF_GBUFFER, 0, np.float32).reshape(h, w, 16)
+        # every fourth column of the view beside the next ones, so that small images see surfaces
+        gbuf = np.ascontiguousarray(np.concatenate([gbuf[:, k::4] for k in range(4)], 1))
+        whole = _trace(ctx, cam, tr, gbuf)[0]
+        assert (whole != 0).any()
+        for x, y in ((512, 512), (519, 505), (1024, 512), (1032, 519), (1024, 576), (1029, 571)):
+            part = _trace(ctx, cam, tr, gbuf[:y, :x])[0]
+            assert np.array_equal(part.view(np.uint32), whole[:y, :x].view(np.uint32)), (x, y)
     finally:
         app.close()

@@ -107,14 +107,23 @@ __global__ __launch_bounds__(448) __attribute__((amdgpu_waves_per_eu(MODE == 0 ?
 }
 
 hipError_t launch_trace(const PyrDesc &pyr, const TraceLaunch &t, hipStream_t s) {
-    // k_trace_split where it is the faster one (us, k_trace / two parts / three
-    // parts).  Isotropic, 8192 tiles: 512x288 94 / 75 / 68, 854x480 183 / 169 /
-    // 160, but 1001x567 FP32 167 / 172 / 178 back to back.  Six directions, 4096
-    // tiles: 384x216 106 / 102 / 105, 640x360 177 / 169 / 178, 854x480 247 / 247 /
-    // 261.  Six parts, without a specular cone to wait for, while six wavefronts
-    // per tile leave SIMDs idle: 128x128 17.6 (three parts 25.2), 256x256 33.0 (32.8).
+    // k_trace_split where it is the faster one.  In us, launch after launch of one view,
+    // k_trace / two / three parts (the room at 64^3, the 2,064 objects at 128^3), with a
+    // specular cone: isotropic up to 8192 tiles, room 640x360 89 / 75 / 73, 960x540 153 /
+    // 146 / 146, 1280x720 246 / 242 / 246, FP32 190 / 185 / 189 and 314 / 315 / 322 at the
+    // last two, objects 640x360 141 / 122 / 126, 960x540 228 / 232 / 242; six directions up
+    // to 4096, room 640x360 146 / 120 / 126, 720x405 168 / 146 / 152, objects 173 / 171 /
+    // 180, 202 / 199 / 207, 960x540 296 / 306 / 319, FP32 640x360 213 / 215 / 222, 960x540
+    // 372 / 389 / 409, FP8 186 / 190 / 196, 334 / 346 / 363.
+    // Where launches of several views overlap, a longest tile costs less and the parts'
+    // set-up more: k_trace is ahead by 1 to 4% at 1001x567 and above.  Without a specular
+    // cone the warped six-direction kernel, which keeps most in scratch, still loses more
+    // by its longest tile up to 9216 tiles (k_trace / two parts: 720x405 198 / 153, 960x540
+    // 259 / 220, 1001x567 273 / 228; overlapping 94.6 / 93.3, 164.3 / 165.5), though no
+    // longer at 1280x720 (overlapping 285.9 / 289.0).  Six parts, while six wavefronts per
+    // tile leave SIMDs idle: room 128x128 isotropic 15 (three parts 22), 256x256 27 (26).
     const int tiles8 = ((t.width + 7) / 8) * ((t.height + 7) / 8);
-    const bool split = tiles8 <= (pyr.aniso ? 4096 : 8192);
+    const bool split = tiles8 <= (!pyr.aniso ? 8192 : (t.warp && !t.enable_reflections ? 9216 : 4096));
     const int parts = pyr.aniso ? 2 : (!t.enable_reflections && tiles8 <= 512 ? 6 : 3);
     const int edge = split ? 8 : 16, run = split ? kSplitRun : kTraceRun;
     const int tiles_x = (t.width + edge - 1) / edge, tiles_y = (t.height + edge - 1) / edge;
