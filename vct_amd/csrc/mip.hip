@@ -6,10 +6,11 @@
 // of the source level (two 4^3 bricks per axis, contiguous 1 KB brick runs) and
 // produces the 4^3, 2^3 and 1^3 blocks of the next three levels: a wavefront per
 // region where the source has one face (k_mip_regions), a workgroup where it has
-// six (k_mip_chain).  So level 0 -- the only large one -- is read exactly once.  Each level is rounded to its storage format before the next one is
-// filtered from it, exactly as a per-level pass over stored texels would be,
-// and the eight taps are summed in the reference's offset order, so the chain
-// is bit-identical to filtering level by level.
+// six or is smaller than a region (k_mip_chain).  So level 0 -- the only large one
+// -- is read exactly once.  Each level is rounded to its storage format before the
+// next one is filtered from it, exactly as a per-level pass over stored texels would
+// be, and the eight taps are summed in the reference's offset order, so the chain is
+// bit-identical to filtering level by level.
 //
 // Anisotropic chains keep six directional volumes per level >= 1 (+x,-x,+y,
 // -y,+z,-z): each is the mean of the four front-to-back composites
@@ -44,11 +45,11 @@ __device__ __forceinline__ float4 round_stage(float4 v, int fp32) {
 }
 
 // One filtering step of the chain: the (cur/2)^3 texels per face of output
-// level k from the cur^3 texels per face in LDS (faces: 1 or 6 source faces).
+// level k from the cur^3 texels per face in LDS (as many source faces as outputs).
 // CUR: cur as a compile-time constant (0: use the argument), which turns the
 // index arithmetic into shifts.
 template <bool ANISO, int CUR>
-__device__ __forceinline__ void mip_step(const MipArgs &a, int cur_rt, int faces, const float4 *in, int in_stride,
+__device__ __forceinline__ void mip_step(const MipArgs &a, int cur_rt, const float4 *in, int in_stride,
                                          float4 *out, int out_stride, int k, int ox, int oy, int oz) {
     constexpr int NF = ANISO ? 6 : 1;
     const int cur = CUR ? CUR : cur_rt;
@@ -79,8 +80,7 @@ __device__ __forceinline__ void mip_step(const MipArgs &a, int cur_rt, int faces
             v.w = v.w * 0.125f;
         } else {
             const int ax = f >> 1, neg = f & 1;
-            const int sf = faces == 1 ? 0 : f;
-            const float4 *src = in + (size_t)sf * in_stride;
+            const float4 *src = in + (size_t)f * in_stride;
             const int oa = ax == 0 ? 1 : 0, ob = ax == 2 ? 1 : 2;
 #pragma unroll
             for (int pa = 0; pa < 2; ++pa)
@@ -157,14 +157,14 @@ __device__ __forceinline__ void mip_step8(const MipArgs &a, const float4 *in, fl
     }
 }
 
-// ANISO: outputs have six faces; SRC6: the source level has six faces (any
-// anisotropic level >= 1).  LDS: the 8^3 source region (per face), then the
-// ping-pong buffers of the three output steps (4^3, 2^3, 1^3 per face).
-template <bool ANISO, bool SRC6>
+// ANISO: source and outputs have six faces.  Without, the source is a level of 2^3
+// or 4^3 texels (a larger one goes to k_mip_regions).  LDS: the 8^3 source region
+// (per face), then the ping-pong buffers of the three output steps (4^3, 2^3, 1^3
+// per face).
+template <bool ANISO>
 __global__ __launch_bounds__(256) void k_mip_chain(MipArgs a) {
     constexpr int NF = ANISO ? 6 : 1;
-    constexpr int SF = SRC6 ? 6 : 1;
-    __shared__ float4 bufA[SF][512];
+    __shared__ float4 bufA[NF][ANISO ? 512 : 64];
     __shared__ float4 bufB[NF][64];
     const int tid = threadIdx.x;
     const int s = a.src.size;
@@ -179,8 +179,8 @@ __global__ __launch_bounds__(256) void k_mip_chain(MipArgs a) {
     const int rx = b % nreg, ry = (b / nreg) % nreg, rz = b / (nreg * nreg);
     const int ox = rx * R, oy = ry * R, oz = rz * R;
     const int R3 = R * R * R;
-    for (int f = 0; f < SF; ++f) {  // the launcher picks SRC6 from the source level's face count
-        if (R == 8 && !a.fp32) {
+    for (int f = 0; f < NF; ++f) {
+        if (ANISO && R == 8 && !a.fp32) {
             // fp16 pairs: the elements of even x hold texels x and x+1; walk
             // brick by brick (32 such elements per brick)
             const int i = tid;  // 256 threads, 256 pair elements
@@ -188,15 +188,14 @@ __global__ __launch_bounds__(256) void k_mip_chain(MipArgs a) {
             const int x = ox + (j & 1) * 4 + (v & 1) * 2;
             const int y = oy + ((j >> 1) & 1) * 4 + ((v >> 1) & 3);
             const int z = oz + (j >> 2) * 4 + (v >> 3);
-            uint4 e = make_uint4(0u, 0u, 0u, 0u);
-            if (!src_zero(a, x, y, z)) e = *(const uint4 *)(a.pyr + a.src.stage + (size_t)elem_index(a.src, x, y, z, f) * 16);
+            const uint4 e = *(const uint4 *)(a.pyr + a.src.stage + (size_t)elem_index(a.src, x, y, z, f) * 16);
             float4 *d = &bufA[f][((z - oz) * R + (y - oy)) * R + (x - ox)];
             d[0] = unpack_h4(e.x, e.y);
             d[1] = unpack_h4(e.z, e.w);
         } else {
             for (int i = tid; i < R3; i += 256) {
                 int x, y, z;
-                if (R == 8) {  // brick-major walk: 8 bricks of 64 contiguous voxels
+                if (ANISO && R == 8) {  // brick-major walk: 8 bricks of 64 contiguous voxels
                     const int j = i >> 6, v = i & 63;
                     x = ox + (j & 1) * 4 + (v & 3);
                     y = oy + ((j >> 1) & 1) * 4 + ((v >> 2) & 3);
@@ -206,27 +205,26 @@ __global__ __launch_bounds__(256) void k_mip_chain(MipArgs a) {
                     y = (i / R) % R;
                     z = i / (R * R);
                 }
-                bufA[f][((z - oz) * R + (y - oy)) * R + (x - ox)] =
-                    src_zero(a, x, y, z) ? make_float4(0.f, 0.f, 0.f, 0.f) : load_stage_texel(a.pyr, a.src, x, y, z, f);
+                bufA[f][((z - oz) * R + (y - oy)) * R + (x - ox)] = load_stage_texel(a.pyr, a.src, x, y, z, f);
             }
         }
     }
     __syncthreads();
-    if (SRC6 && R == 8) {  // the three steps with their sizes known at compile time
+    if (ANISO && R == 8) {  // the three steps with their sizes known at compile time
         mip_step8(a, &bufA[0][0], &bufB[0][0], ox, oy, oz);
         if (a.nout > 1) {
             __syncthreads();
-            mip_step<ANISO, 4>(a, 4, NF, &bufB[0][0], 64, &bufA[0][0], 8, 1, ox, oy, oz);
+            mip_step<ANISO, 4>(a, 4, &bufB[0][0], 64, &bufA[0][0], 8, 1, ox, oy, oz);
         }
         if (a.nout > 2) {
             __syncthreads();
-            mip_step<ANISO, 2>(a, 2, NF, &bufA[0][0], 8, &bufB[0][0], 64, 2, ox, oy, oz);
+            mip_step<ANISO, 2>(a, 2, &bufA[0][0], 8, &bufB[0][0], 64, 2, ox, oy, oz);
         }
         return;
     }
-    int cur = R, faces = SF;
+    int cur = R;
     float4 *in = &bufA[0][0];
-    int in_stride = 512;
+    int in_stride = ANISO ? 512 : 64;
     for (int k = 0; k < a.nout; ++k) {
         const int d = cur >> 1;
         if (d < 1) break;
@@ -234,12 +232,11 @@ __global__ __launch_bounds__(256) void k_mip_chain(MipArgs a) {
         // bufA (k odd, <= 2^3 per face)
         float4 *out = (k & 1) ? &bufA[0][0] : &bufB[0][0];
         const int out_stride = (k & 1) ? 8 : 64;
-        mip_step<ANISO, 0>(a, cur, faces, in, in_stride, out, out_stride, k, ox, oy, oz);
+        mip_step<ANISO, 0>(a, cur, in, in_stride, out, out_stride, k, ox, oy, oz);
         __syncthreads();
         in = out;
         in_stride = out_stride;
         cur = d;
-        faces = NF;
     }
 }
 
@@ -620,9 +617,8 @@ hipError_t launch_mip(const PyrDesc &pyr, hipStream_t s) {
         } else if (R == 8 && S.nfaces == 1) {
             if (fp32) hipLaunchKernelGGL((k_mip_regions<false, true>), wgrid, dim3(256), 0, s, a);
             else hipLaunchKernelGGL((k_mip_regions<false, false>), wgrid, dim3(256), 0, s, a);
-        } else if (pyr.aniso && S.nfaces == 6) hipLaunchKernelGGL((k_mip_chain<true, true>), grid, dim3(256), 0, s, a);
-        else if (pyr.aniso) hipLaunchKernelGGL((k_mip_chain<true, false>), grid, dim3(256), 0, s, a);
-        else hipLaunchKernelGGL((k_mip_chain<false, false>), grid, dim3(256), 0, s, a);
+        } else if (pyr.aniso) hipLaunchKernelGGL(k_mip_chain<true>, grid, dim3(256), 0, s, a);
+        else hipLaunchKernelGGL(k_mip_chain<false>, grid, dim3(256), 0, s, a);
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
         src += nout;
