@@ -22,8 +22,10 @@ __device__ __forceinline__ int xcd_group(int run) {
 // time, which the scalar data cache they share rewards (a workgroup whose
 // wavefronts take different cones of one tile misses it three times as often).
 // Six wavefronts per SIMD (five for the formats of one texel per element) at
-// the price of registers kept in scratch between cones: 490 -> 467 us for the
-// 1280x720 six-direction gather.  With reflections the grid holds every tile
+// the price of registers kept in scratch between cones (with six directions 16 to
+// 27 of a lane's, 64 to 96 bytes; isotropic at most 6): 490 -> 467 us for the
+// 1280x720 six-direction gather, though 162 of the 229 MB that a 1920x1080 launch
+// writes are scratch.  With reflections the grid holds every tile
 // twice, first its specular cones (the longer and less even half), then its
 // diffuse cones: shorter wavefronts leave a shorter tail (574 -> 529 us for that
 // gather by itself).  The whole of it, against one contiguous band of tiles per

@@ -56,8 +56,8 @@ __device__ __forceinline__ uint4 bload16(__amdgpu_buffer_rsrc_t r, uint32_t off)
 // Scalar load of 16 bytes at a wave-uniform offset: through the constant
 // address space the load becomes s_load_dwordx4 into SGPRs (scalar data cache,
 // not the vector memory pipeline).  The pyramid is not written while a trace
-// runs.  The offset is one the vector path would load (clamped texel indices),
-// so it is inside the allocation.
+// runs.  Nothing checks the offset (bload16's descriptor has the size): the callers'
+// indices keep it inside the allocation.
 typedef __attribute__((address_space(4))) const char cchar;
 __device__ __forceinline__ uint4 sload16(const char *pyr, uint32_t off) {
     const u32x4 v = *(const __attribute__((address_space(4))) u32x4 *)((cchar *)pyr + off);
@@ -180,7 +180,13 @@ __device__ __forceinline__ void axis_terms_s(uint32_t i, uint32_t mul, uint32_t 
 // acc += lw * (trilinear sample of level l at p): isotropic, or the
 // dir^2-weighted mix of the three faces that face the cone.  l is wave-uniform.
 // The border bricks hold texels -1 and s as zeros, so no index is clamped and
-// no weight masked; indices are shifted by one brick (+4).  Returns
+// no weight masked; indices are shifted by one brick (+4).  What that rests on: p is
+// in [0, 1] up to a few roundings.  A march leaves the box before it samples; a warped
+// position is a convex mix of the warp texture's unorm16 texels, and 1 + 2^-20 still
+// floors to texel s - 1 of 512.  So a shifted index is in 3 .. s + 3 and its upper
+// neighbour at most s + 4, the first texel of the border brick; both are below 2^10.
+// A position that is not a number passes the march's comparisons: the conversion to
+// int (v_cvt_i32_f32) makes 0 of it, index 4.  Returns
 // (wave-uniform) whether every texel fetched, in every lane, was +0 (ZQ: also
 // test the per-lane fetches, which costs vector instructions).  An fp8 level
 // reports false: its codes underflow, so a zero there does not say that the
@@ -193,8 +199,7 @@ __device__ __forceinline__ void axis_terms_s(uint32_t i, uint32_t mul, uint32_t 
 // path, without its vector memory traffic.  Whether they do is decided on the
 // packed cell indices, before any address exists: the addresses of a shared
 // cell are scalar arithmetic, and its weights are formed only if one of the
-// cell's texels is not zero.  What bounds the trace is VALU issue (95% of the
-// cycles at 1080p): an empty shared cell costs 12 vector instructions (60 when
+// cell's texels is not zero.  What bounds the trace is VALU issue: an empty shared cell costs 12 vector instructions (60 when
 // addresses and weights were formed first), an occupied one 32 plus 36 a face.
 // Texels are weighted and summed in one fixed order: a march compares its
 // opacity with 0.95, and sums that differ in the last bit end some cones a step
