@@ -43,12 +43,12 @@ PEAK_HBM_GBS = 8000.0
 #    x1 (profiles/counters_copy_calibration.md).  The read factor comes from a
 #    copy's 128-byte requests, so for smaller requests the read bytes are an
 #    upper bound.
-#  - instruction issue: SQ_INSTS_VALU per wavefront and SQ_ACTIVE_INST_VALU x 4
-#    / (1024 SIMDs x kernel cycles) -- the fraction of SIMD cycles issuing VALU,
-#    the ceiling this kernel actually runs against.
+#  - instruction issue: SQ_INSTS_VALU per wavefront and SQ_INSTS_VALU x 4 /
+#    (1024 SIMDs x kernel cycles) -- how full the instruction issue is that this
+#    kernel runs against (no share of a peak: other kernels pass 1).
 TRACE_PROFILE = "profiles/counters_trace_scalar_path.md"
-TRACE_FETCH_KIB, TRACE_WRITE_KIB = 184649, 223412
-TRACE_VALU_PER_WAVE, TRACE_VALU_BUSY = 9654, 0.80
+TRACE_FETCH_KIB, TRACE_WRITE_KIB = 183987, 219558
+TRACE_VALU_PER_WAVE, TRACE_VALU_BUSY = 9667, 0.83
 METRIC = "ms/frame voxelize+inject+mip+trace @256^3,1080p; GB/s vs peak; learned vs plain"
 
 

@@ -24,7 +24,7 @@ __device__ __forceinline__ int xcd_group(int run) {
 // Six wavefronts per SIMD (five for the formats of one texel per element) at
 // the price of registers kept in scratch between cones (with six directions 16 to
 // 27 of a lane's, 64 to 96 bytes; isotropic at most 6): 490 -> 467 us for the
-// 1280x720 six-direction gather, though 162 of the 229 MB that a 1920x1080 launch
+// 1280x720 six-direction gather, though 158 of the 225 MB that a 1920x1080 launch
 // writes are scratch.  With reflections the grid holds every tile
 // twice, first its specular cones (the longer and less even half), then its
 // diffuse cones: shorter wavefronts leave a shorter tail (574 -> 529 us for that
